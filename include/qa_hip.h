@@ -589,6 +589,15 @@ int qa_d_quantize_nhwc(const float* x, int64_t N, int64_t C, int64_t HW,
                        int64_t zp, int64_t qmin, int64_t qmax, int64_t so,
                        void* stream);
 
+/* Dequantizes channels-last storage (int8 or int16; element (n, c, pixel) at
+ * x + n*x_sn + c + pixel*x_sp, x_sp >= C) into a dense float32 NCHW tensor,
+ * (float)((stored + in_so - zp) * scale) as qa_d_dequantize_f32 (a graph
+ * output; the reference: quant_container.py:186-192). */
+int qa_d_dequantize_nchw(const void* x, int in_code, int64_t x_sn,
+                         int64_t x_sp, int64_t N, int64_t C, int64_t HW,
+                         float* y, double scale, int64_t zp, int64_t in_so,
+                         void* stream);
+
 /* Quantizes float32 NCHW input [N, C, H, W] (C <= 4) into the int8 rows of
  * a convolution whose stride equals its kernel KH x KW (no padding; KW a
  * multiple of 4, H and W multiples of the kernel; 16-byte aligned x and

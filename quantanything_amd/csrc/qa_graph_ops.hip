@@ -10,6 +10,14 @@
 
 #include "qa_common.h"
 
+namespace qa {
+// Graph input in any other pixel stride or storage (qa_layout.hip).
+bool launch_quantize_planes(const float* x, int64_t N, int64_t C, int64_t HW,
+                            void* y, int y_code, int64_t y_sp, double scale,
+                            int64_t zp, int64_t qmin, int64_t qmax,
+                            int64_t so, hipStream_t st);
+}  // namespace qa
+
 namespace {
 
 constexpr int kThreads = 256;
@@ -190,36 +198,24 @@ __global__ __launch_bounds__(kThreads) void k_quantize_patches(
     }
 }
 
-// Graph input: float32 NCHW -> quantized channels-last with pixel stride
-// y_sp >= C (padding channels written as 0), one thread per pixel.
-template <class TOut>
-__global__ __launch_bounds__(kThreads) void k_quantize_cl(
+// Graph input of at most 4 channels, int8 with 4 bytes a pixel: one word a
+// pixel and thread (HW not a multiple of 4).
+__global__ __launch_bounds__(kThreads) void k_quantize_cl4(
     const float* __restrict__ x, int64_t N, int64_t C, int64_t HW,
-    TOut* __restrict__ y, int64_t y_sp, double scale, double inv, int64_t zp,
-    int64_t qmin, int64_t qmax, int64_t so, int word) {
+    int8_t* __restrict__ y, double scale, double inv, int64_t zp,
+    int64_t qmin, int64_t qmax, int64_t so) {
     const int64_t total = N * HW;
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * kThreads) {
         const int64_t n = i / HW, p = i - n * HW;
-        TOut* dst = y + i * y_sp;
-        if (word) {  // int8, 4 bytes a pixel, aligned: one word store
-            uint32_t w = 0;
-            for (int64_t c = 0; c < C; ++c)
-                w |= (uint32_t)(uint8_t)(qa_quantize_one_fast(
-                                             x[(n * C + c) * HW + p], scale,
-                                             inv, zp, qmin, qmax) -
-                                         so)
-                     << (8 * c);
-            *(uint32_t*)dst = w;
-            continue;
-        }
-        for (int64_t c = 0; c < y_sp; ++c) {
-            int64_t v = 0;
-            if (c < C)
-                v = qa_quantize_one_fast(x[(n * C + c) * HW + p], scale, inv,
-                                         zp, qmin, qmax) - so;
-            dst[c] = (TOut)v;
-        }
+        uint32_t w = 0;
+        for (int64_t c = 0; c < C; ++c)
+            w |= (uint32_t)(uint8_t)(qa_quantize_one_fast(
+                                         x[(n * C + c) * HW + p], scale, inv,
+                                         zp, qmin, qmax) -
+                                     so)
+                 << (8 * c);
+        *(uint32_t*)(y + i * 4) = w;
     }
 }
 
@@ -612,25 +608,27 @@ QA_API int qa_d_quantize_nhwc(const float* x, int64_t N, int64_t C,
         return -1;
     }
     hipStream_t st = (hipStream_t)stream;
-    const unsigned g = qa::grid_1d(N * HW, kThreads, 1 << 20);
-    const double inv = 1.0 / scale;
-    const int word = y_code == 1 && y_sp == 4 && (uintptr_t)y % 4 == 0;
-    if (word && C <= 4 && HW % 4 == 0 && (uintptr_t)y % 16 == 0 &&
-        (uintptr_t)x % 16 == 0) {
-        const unsigned g4 = qa::grid_1d(N * HW / 4, kThreads, 2048);
-        k_quantize_cl4x4<<<g4, kThreads, 0, st>>>(
-            x, N, C, HW, (int8_t*)y, scale, inv, zp, qmin, qmax, so);
-    } else if (y_code == 1)
-        k_quantize_cl<int8_t><<<g, kThreads, 0, st>>>(
-            x, N, C, HW, (int8_t*)y, y_sp, scale, inv, zp, qmin, qmax, so,
-            word);
-    else if (y_code == 2)
-        k_quantize_cl<int16_t><<<g, kThreads, 0, st>>>(
-            x, N, C, HW, (int16_t*)y, y_sp, scale, inv, zp, qmin, qmax, so,
-            0);
-    else {
+    if (y_code != 1 && y_code != 2) {
         qa::set_error("qa_d_quantize_nhwc", "storage must be int8 or int16");
         return -1;
+    }
+    const double inv = 1.0 / scale;
+    if (y_code == 1 && y_sp == 4 && (uintptr_t)y % 4 == 0) {
+        // 4 bytes a pixel (image stems): one word a pixel, four pixels a
+        // thread where the planes are float4s
+        if (HW % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)x % 16 == 0)
+            k_quantize_cl4x4<<<qa::grid_1d(N * HW / 4, kThreads, 2048),
+                               kThreads, 0, st>>>(
+                x, N, C, HW, (int8_t*)y, scale, inv, zp, qmin, qmax, so);
+        else
+            k_quantize_cl4<<<qa::grid_1d(N * HW, kThreads, 1 << 20),
+                             kThreads, 0, st>>>(
+                x, N, C, HW, (int8_t*)y, scale, inv, zp, qmin, qmax, so);
+    } else {
+        return qa::launch_quantize_planes(x, N, C, HW, y, y_code, y_sp, scale,
+                                          zp, qmin, qmax, so, st)
+                   ? 0
+                   : -1;
     }
     return launched("qa_d_quantize_nhwc") ? 0 : -1;
 }

@@ -681,6 +681,18 @@ class DeviceExecutor:
                                         "qa_d_conv")))
         for name in g.outputs:
             t = self.tensors[name]
+            if len(t.shape) == 4 and t.nhwc and t.sc == 1 and \
+                    t.sp >= t.channels and name not in self.softmax_of and \
+                    t.shape[0] * t.pixels < 2**31 - 4096:
+                # channels-last: dequantized into NCHW floats in one launch
+                yf = torch.empty(t.shape, dtype=torch.float32, device="cuda")
+                self.outputs_f32[name] = yf
+                self._add(f"dequantize:{name}", lambda s, t=t, yf=yf:
+                          _ok(self.lib.qa_d_dequantize_nchw(
+                              t.ptr, t.code, t.sn, t.sp, t.shape[0],
+                              t.channels, t.pixels, yf.data_ptr(),
+                              t.qp.scale, t.qp.zp, t.so, s), "dequantize"))
+                continue
             if not (t.contiguous_2d() or (t._strides is not None and
                                           t.row_major())):
                 # a dense copy that the dequantization reads

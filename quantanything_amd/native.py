@@ -111,6 +111,8 @@ def _declare(lib):
         "qa_d_quantize_f32": (i32, [p, p, i32, i64, f64, i64, i64, i64, i64,
                                     p]),
         "qa_d_dequantize_f32": (i32, [p, i32, p, i64, f64, i64, i64, p]),
+        "qa_d_dequantize_nchw": (i32, [p, i32] + [i64] * 5 + [p, f64, i64,
+                                       i64, p]),
         "qa_d_pad_nd": (i32, [p, p]),
         "qa_d_maxpool": (i32, [p, p]),
         "qa_d_fb_binary": (i32, [p, p]),
