@@ -51,7 +51,8 @@ struct ConvArgs {
     // ---- packed int8 weights (MFMA path) ----
     const int8_t* wp;
     const int8_t* wfrag;            // the same in fragment order, or NULL
-    int32_t layout;                 // 0 tap-major 16-channel groups, 1 stem
+    int32_t layout;                 // 0 tap-major 16-channel groups, 1 stem,
+                                    // 2 depthwise
     int32_t CB, KG, KGp, Kreal;
     uint64_t mg_cb, mg_kw;          // ceil(2^32 / CB), ceil(2^32 / KW)
     int32_t st_dn, st_doy, st_dox;  // a wave's pixel stride as (n, oy, ox)
@@ -188,6 +189,10 @@ bool mfma_launch_lds(const ConvArgs& b, int wm, bool split, int epi,
 bool mfma_launch_l2(const ConvArgs& b, int wm, bool split, int epi,
                     hipStream_t st);
 bool launch_conv_valu(const ConvArgs& a, hipStream_t st);
+// Depthwise convolutions (layout 2; qa_conv_dw.hip); arguments in launch
+// form, `epi` as chosen by launch_conv_mfma.
+bool conv_dw_applies(const ConvArgs& b);
+bool launch_conv_dw(const ConvArgs& b, int epi, hipStream_t st);
 // Large GEMM descriptors (H = W = 1, K a multiple of 64) with the int8 table
 // epilogue on 128 x 128 blocks (qa_gemm_big.hip); `epi` as chosen by
 // launch_conv_mfma.

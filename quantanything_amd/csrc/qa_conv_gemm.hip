@@ -178,6 +178,12 @@ void set_geometry(ConvArgs& a, int64_t N, int64_t C, int64_t H, int64_t W,
 void pack_geometry(int64_t Cout, int64_t Cg, int64_t KH, int64_t KW,
                    int64_t G, int layout, int64_t* CB, int64_t* KG,
                    int64_t* KGp, int64_t* rows) {
+    if (layout == 2) {  // depthwise: a row of KH*KW bytes a channel
+        *CB = 1;
+        *KG = *KGp = std::max<int64_t>(1, ceil_div(KH * KW, 16));
+        *rows = round_up(std::max<int64_t>(Cout, 1), 16);
+        return;
+    }
     // layout 1: CB groups of 4 kernel columns per kernel row
     *CB = layout == 1 ? ceil_div(std::max<int64_t>(KW, 1), 4)
                       : ceil_div(Cg, 16);
@@ -213,8 +219,39 @@ bool mfma_grid_ok(int64_t Cog, int64_t G) {
 int pack_weights(const int32_t* w, int64_t Cout, int64_t Cg, int64_t KH,
                  int64_t KW, int64_t G, int64_t a_off, int layout, int8_t* wp,
                  int64_t* corr, int32_t* boff, int32_t* needs_rowsum) {
-    if (G <= 0 || Cout % G || Cg < 0 || (layout == 1 && (Cg > 4 || KW > 16)))
+    if (G <= 0 || Cout % G || Cg < 0 ||
+        (layout == 1 && (Cg > 4 || KW > 16)) ||
+        (layout == 2 && (Cg != 1 || Cout != G)))
         return -1;
+    if (layout == 2) {
+        // one row a channel; the sums an offset needs are those of the
+        // channel's own window
+        const int64_t K = KH * KW;
+        int64_t CB, KG, KGp, rows;
+        pack_geometry(Cout, Cg, KH, KW, G, layout, &CB, &KG, &KGp, &rows);
+        memset(wp, 0, (size_t)(rows * KGp * 16));
+        int32_t any = 0;
+        for (int64_t co = 0; co < Cout; ++co) {
+            int lo = 0, hi = 0;
+            for (int64_t k = 0; k < K; ++k) {
+                lo = std::min(lo, w[co * K + k]);
+                hi = std::max(hi, w[co * K + k]);
+            }
+            if ((int64_t)hi - lo > 255) return 1;
+            const int b = (lo >= -128 && hi <= 127) ? 0 : lo + 128;
+            if (b) any = 1;
+            int64_t colsum = 0;
+            for (int64_t k = 0; k < K; ++k) {
+                const int v = w[co * K + k] - b;
+                wp[co * KGp * 16 + k] = (int8_t)v;
+                colsum += v;
+            }
+            corr[co] = a_off * colsum + K * a_off * (int64_t)b;
+            boff[co] = b;
+        }
+        *needs_rowsum = any;
+        return 0;
+    }
     const int64_t Cog = Cout / G;
     int64_t CB, KG, KGp, rows;
     pack_geometry(Cout, Cg, KH, KW, G, layout, &CB, &KG, &KGp, &rows);
@@ -516,12 +553,14 @@ QA_API void qa_conv_i32_i32_i64(const int32_t* x, const int32_t* w,
 QA_API int64_t qa_pack_weights_i8_size(int64_t Cout, int64_t Cg, int64_t KH,
                                        int64_t KW, int64_t G, int64_t layout,
                                        int64_t* kgp, int64_t* rows_per_group) {
-    if (G <= 0 || Cout < 0 || Cout % G || layout < 0 || layout > 1) return -1;
+    if (G <= 0 || Cout < 0 || Cout % G || layout < 0 || layout > 2 ||
+        (layout == 2 && (Cg != 1 || Cout != G)))
+        return -1;
     int64_t CB, KG, KGp, rows;
     pack_geometry(Cout, Cg, KH, KW, G, (int)layout, &CB, &KG, &KGp, &rows);
     if (kgp) *kgp = KGp;
     if (rows_per_group) *rows_per_group = rows;
-    return G * rows * KGp * 16;
+    return (layout == 2 ? 1 : G) * rows * KGp * 16;
 }
 
 QA_API int qa_pack_weights_i8(const int32_t* w, int64_t Cout, int64_t Cg,
@@ -690,7 +729,8 @@ int desc_args(const qa_conv_desc* d, ConvArgs& a, const char* who) {
                    d->G == 1)
                 : (xa % 16 == 0 && d->x_sn % 16 == 0 &&
                    (d->H * d->W == 1 || d->x_sp % 16 == 0) &&
-                   (d->G == 1 || (d->C / d->G) % 16 == 0));
+                   (d->G == 1 || (d->C / d->G) % 16 == 0 ||
+                    d->w_layout == 2));
         if (d->x_code != 1 || d->x_sc != 1 || d->x_add < -127 ||
             d->x_add > 128 || d->w_kgp != KGp || d->w_rows != rows ||
             a.Kreal >= 131072 || !aligned) {
@@ -704,7 +744,7 @@ int desc_args(const qa_conv_desc* d, ConvArgs& a, const char* who) {
         a.KG = (int32_t)KG;
         a.KGp = (int32_t)KGp;
         a.wp_rstride = KGp * 16;
-        a.wp_gstride = rows * KGp * 16;
+        a.wp_gstride = d->w_layout == 2 ? KGp * 16 : rows * KGp * 16;
         a.pad_value = (int32_t)(-d->x_add);
         a.rowsum = (int32_t)d->needs_rowsum;
         a.plan = d->epi_plan;

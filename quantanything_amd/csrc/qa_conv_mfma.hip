@@ -26,7 +26,8 @@ int fast_io_args(const ConvArgs& a, ConvArgs& b, int epi) {
                    (sc == 1 && (ohw == 1 || sn == ohw * sp) &&
                     pst(sn, sp) % 4 == 0 && (uintptr_t)p % 4 == 0);
         };
-        b.fastio = a.mode == EPI_QUANT && (a.G == 1 || a.Cog % 4 == 0) &&
+        b.fastio = a.mode == EPI_QUANT &&
+                   (a.G == 1 || a.Cog % 4 == 0 || a.layout == 2) &&
                    dense(a.y, a.y_sn, a.y_sc, a.y_sp) &&
                    dense(a.res, a.res_sn, a.res_sc, a.res_sp) &&
                    dense(a.y2, a.y2_sn, a.y2_sc, a.y2_sp);
@@ -47,6 +48,15 @@ int fast_io_args(const ConvArgs& a, ConvArgs& b, int epi) {
 // even 16-channel blocks leave most SIMDs idle.
 bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
     if (a.M <= 0 || a.Cog <= 0 || a.G <= 0) return true;
+    if (a.layout == 2) {
+        ConvArgs b;
+        if (a.mode != EPI_QUANT || a.y_code != 1) {
+            set_error("launch_conv_mfma", "int8 output expected");
+            return false;
+        }
+        const int epi = fast_io_args(a, b, Q8_GENERAL);
+        return launch_conv_dw(b, epi, st);
+    }
     if (a.M >= ((int64_t)1 << 31) || a.KGp < 4 || (a.KGp & 3) ||
         a.KGp >= (1 << 16) || a.CB < 1 || a.KW < 1 ||
         (int64_t)(a.KH - 1) * a.DH >= 32768 ||

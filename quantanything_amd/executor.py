@@ -725,7 +725,8 @@ class DeviceExecutor:
                 off_bytes % 4 == 0
         pix = x.pixels if len(x.shape) == 4 else 1
         return off_bytes % 16 == 0 and x.sn % 16 == 0 and \
-            (pix == 1 or x.sp % 16 == 0) and (groups == 1 or cg % 16 == 0)
+            (pix == 1 or x.sp % 16 == 0) and \
+            (groups == 1 or cg % 16 == 0 or layout == 2)
 
     @staticmethod
     def _f64_ok(x, a_off):
@@ -829,6 +830,12 @@ class DeviceExecutor:
                    pads[0], pads[1], dil[0], dil[1], groups, oh, ow)
             layout = 1 if (groups == 1 and cg <= 4 and kw <= 16 and
                            x.sp == 4) else 0
+            if cg == 1 and groups == cin == cout and groups > 1 and \
+                    kh * kw <= 52 and x.sp >= -(-cout // 16) * 16 and \
+                    (h + pads[0] + kh * dil[0]) * \
+                    (w + pads[1] + kw * dil[1]) * x.sp < 2**30 and \
+                    max((kh - 1) * dil[0], (kw - 1) * dil[1]) < 32768:
+                layout = 2  # depthwise (the kernel's 32-bit offsets)
         else:
             k, ncol = layer.w_centered.shape
             xv = x.rows_view()
@@ -2201,6 +2208,8 @@ class DeviceExecutor:
         re-checks the LDS size), the large-GEMM kernel and the narrow-GEMM
         kernel where their shapes apply."""
         cog = d.Cout // d.G
+        if d.w_code == 1 and d.w_layout == 2:
+            return [0]  # depthwise: one kernel
         if d.w_code == 8:  # FP64 path: wm | tm << 4 | split << 8
             wm_max = 1 if cog <= 16 else 2 if cog <= 32 else 4
             out = [0] + [0x10000 | c for c in F64_TILES if c & 15 <= wm_max]
