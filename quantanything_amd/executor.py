@@ -92,6 +92,7 @@ class DeviceTensor:
         self.shape = tuple(int(s) for s in shape)
         self.sn, self.sc, self.sp = int(sn), int(sc), int(sp)
         self.code, self.so, self.qp = code, int(so), qp
+        self.zero_pad = False  # bytes between a row and the next are 0
         self._strides = None if strides is None else \
             tuple(int(v) for v in strides)
         self.nhwc = True
@@ -522,6 +523,32 @@ class DeviceExecutor:
                         for k in range(len(shape)))
         return DeviceTensor.nd(buf, 0, shape, strides, self.code, self.so, qp)
 
+    def _new_rows(self, name, shape, qp):
+        """A 2-D tensor ``name`` read by Gemms alone: int8 rows padded with
+        zeros to the 64-byte K-steps of the GEMM kernels (a dense tensor
+        otherwise, or where other readers may want it dense)."""
+        users = self._cons.get(name, [])
+        if self.code != 1 or name in self.graph.outputs or not users or \
+                any(u.kind != "gemm" for u in users) or shape[1] % 64 == 0:
+            return self._new(shape, qp)
+        return self._padded_rows(shape, qp)
+
+    def _padded_rows(self, shape, qp):
+        m, k = shape
+        ks = -(-k // 64) * 64
+        buf = torch.zeros(m * ks + TAIL, dtype=self.dtype, device="cuda")
+        t = DeviceTensor(buf, 0, (m, k), ks, 1, 0, self.code, self.so, qp)
+        t.zero_pad = True
+        return t
+
+    def _aligned(self, name, x):
+        """``x`` (a matrix, or channels-last) copied to where the int8 MFMA
+        kernels can read it: rows or pixels on 16-byte boundaries."""
+        y = self._padded_rows(x.shape, x.qp) if len(x.shape) == 2 else \
+            self._new(x.shape, x.qp)
+        self._copy(name, x, y)
+        return y
+
     def _copy(self, name, x, y, mode=0, rescale=None, requant=None):
         """Launch copying x into the view y (same logical shape): mode 0
         unchanged, 1 integer rescale ``(zp_in, m, s, zp_out, qmin, qmax)``,
@@ -580,6 +607,11 @@ class DeviceExecutor:
     # ------------------------------------------------------------ planning --
     def _plan(self, input_shapes):
         c, g = self.c, self.graph
+        cons = {}
+        for l in c.layers:
+            for i in l.data_inputs:
+                cons.setdefault(i, []).append(l)
+        self._cons = cons
         for name, shape in input_shapes.items():
             qp = c.qparams[name]
             shape = tuple(shape)
@@ -595,6 +627,14 @@ class DeviceExecutor:
                                   xf.data_ptr(), n, ch, hw, t.ptr, t.code,
                                   t.sp, qp.scale, qp.zp, qp.qmin, qp.qmax,
                                   t.so, s), "quantize"))
+            elif len(shape) == 2 and (t := self._new_rows(name, shape,
+                                                          qp)).zero_pad:
+                # rows as one-pixel images: the padding is written as 0
+                self._add(f"quantize:{name}", lambda s, xf=xf, t=t, qp=qp:
+                          _ok(self.lib.qa_d_quantize_nhwc(
+                              xf.data_ptr(), t.shape[0], t.shape[1], 1, t.ptr,
+                              t.code, t.sn, qp.scale, qp.zp, qp.qmin,
+                              qp.qmax, t.so, s), "quantize"))
             else:
                 t = self._new(shape, qp)
                 numel = xf.numel()
@@ -617,11 +657,6 @@ class DeviceExecutor:
 
         layers = c.layers
         producer = g.producer_index()
-        cons = {}
-        for l in layers:
-            for i in l.data_inputs:
-                cons.setdefault(i, []).append(l)
-        self._cons = cons
         absorbed = set()
         for layer in layers:
             if layer.name in absorbed:
@@ -849,8 +884,10 @@ class DeviceExecutor:
             groups, cg, kh, kw, cout = 1, k, 1, 1, ncol
             layout = 0
             # rows of the input as images of one pixel
+            zero_pad = x.zero_pad
             x = DeviceTensor(x.buf, x.offset, (m, k), xv[2], 1, 0, x.code,
                              x.so, x.qp)
+            x.zero_pad = zero_pad
         if layer.kind == "conv" and (not x.nhwc or x.sc != 1):
             # rows and columns strided apart (a Slice with a step) or
             # channels not contiguous (a dense copy): the view copied into
@@ -859,7 +896,22 @@ class DeviceExecutor:
             self._copy(f"copy:{layer.name}", x, xc)
             x = xc
         use_mfma = self._mfma_ok(layer, x, layout, groups, cg, cg * kh * kw)
+        if not use_mfma and x.code == 1 and x.sc == 1 and layout != 1 and \
+                (len(x.shape) == 2 or x.channels > 4):
+            # rows or pixels off the 16-byte grid (odd features, channel
+            # halves): one copy onto it, where nothing else is in the way
+            probe = DeviceTensor(None, 0, (1, 16, 1, 1), 16, 1, 16, x.code,
+                                 x.so, x.qp)
+            if self._mfma_ok(layer, probe, layout, groups, cg,
+                             cg * kh * kw) and self._weights_dev(
+                                 layer, x, layout, True)["w_code"] == 1:
+                x = self._aligned(f"copy:{layer.name}", x)
+                use_mfma = True
         info = self._weights_dev(layer, x, layout, use_mfma)
+        if layer.kind == "gemm" and x.zero_pad and info["w_code"] == 1 and \
+                info["kgp"] * 16 <= x.sn:
+            # whole 64-byte K-steps: the padding meets zero weights
+            geo = (geo[0], info["kgp"] * 16) + geo[2:]
         (d.N, d.C, d.H, d.W, d.Cout, d.KH, d.KW, d.SH, d.SW, d.PH, d.PW,
          d.DH, d.DW, d.G, d.OH, d.OW) = geo
         d.x, d.x_code = x.ptr, x.code
@@ -890,8 +942,11 @@ class DeviceExecutor:
             d.lut_offset = lut_layer.lut_offset
             d.lut_len = len(lut_layer.lut)
             final_qp = lut_layer.out_qp[0]
-        y = self._new(out_shape, final_qp,
-                      dense=layer.kind == "gemm" and len(out_shape) != 2)
+        if layer.kind == "gemm" and len(out_shape) == 2:
+            y = self._new_rows((add_layer or lut_layer or
+                                layer).node.outputs[0], out_shape, final_qp)
+        else:
+            y = self._new(out_shape, final_qp, dense=layer.kind == "gemm")
         if add_layer is not None:
             rname, first = res
             r = self.tensors[rname]
