@@ -25,7 +25,7 @@
 // l%16.
 #include <type_traits>
 
-#include "qa_conv_mfma.h"
+#include "qa_conv_bs.h"
 
 namespace qa {
 namespace {
@@ -128,44 +128,6 @@ __device__ __forceinline__ void f64_store(const ConvArgs& a, int64_t co,
     const int64_t q = quant_one(a, v + pre, m, s, rq);
     store_any(a.y, a.y_code, yi, q - a.y_so);
     if (a.y2) store_any(a.y2, a.y_code, y2i, rescale2(a, q) - a.y_so);
-}
-
-// The 128-bit requantization of one value (out of line: the float64 form
-// below hands it the rare values it cannot decide).
-__device__ __noinline__ int64_t requant_exact(int64_t x, int64_t m, int64_t s,
-                                              int64_t zp, int64_t lo,
-                                              int64_t hi) {
-    return qa_clip128(qa_mbqm_fast(x, m, s) + zp, lo, hi);
-}
-
-// Exact float64 forms of the fixed-point multiplies of the 16-bit epilogue
-// (qa_mbqm: floor(x m 2^-ts + 1/2), ts = 31 + shift):
-//  * requantize, |x| < 2^53, |m| < 2^31, 1 <= ts <= 120, clip bounds within
-//    2^19: y = fma(x, m 2^-ts, 1/2 + zp) is one rounding of the exact value
-//    (x and m 2^-ts are exact doubles), |error| <= 2^-52 |y|; below |y| =
-//    2^20, floor(y) is the exact result unless frac(y) lies within 2^-30 of
-//    0 or 1 (those values take requant_exact); above, the clip gives the
-//    same bound either way.
-//  * multiplies of a clipped value (|d| < 2^20) by |m| < 2^31 with 1 <= ts
-//    <= 53 (the residual Add, the rescaled copy): d m is an exact double
-//    below 2^51, and so is d m 2^-ts + 1/2, so floor gives the exact result.
-struct MulD {
-    double md;
-    bool ok;
-};
-__device__ __forceinline__ MulD mul_d(int64_t m, int64_t shift, int64_t tmax) {
-    const int64_t ts = 31 + shift;
-    MulD r;
-    r.ok = ts >= 1 && ts <= tmax && m > -((int64_t)1 << 31) &&
-           m < ((int64_t)1 << 31);
-    r.md = r.ok ? ldexp((double)m, -(int)ts) : 0.0;
-    return r;
-}
-__device__ __forceinline__ double round_d(double d, double md) {
-    return floor(fma(d, md, 0.5));
-}
-__device__ __forceinline__ double clamp_d(double v, int64_t lo, int64_t hi) {
-    return fmin(fmax(v, (double)lo), (double)hi);
 }
 
 // The epilogue of NV exact sums v[j] of one output channel co at pixels
@@ -706,6 +668,17 @@ bool launch_conv_f64(const ConvArgs& a, hipStream_t st) {
         if (a.tile_hint & TILE_VALID) code = a.tile_hint & 0xffff;
         // the narrow form has one 16-channel block a wave
         const bool nform = narrow && a.Cg % 16 != 0;
+        // the weights in LDS, wherever they fit (a tile code of this form
+        // gives the channel block; one tile a wave)
+        if ((code & 0xff00) == 0x1000 && conv_bsl_applies(b)) {
+            const bool hint = (a.tile_hint & TILE_VALID) != 0;
+            const int hw = code & 15;
+            return launch_conv_bsl(b, nform,
+                                   hint && (hw == 1 || hw == 2 || hw == 4)
+                                       ? hw
+                                       : 0,
+                                   st);
+        }
         if (nform && (code & 0xff00) == 0x1000) code = (code & ~15) | 1;
         const int wm = code & 15, tm = (code >> 4) & 15;
         if ((code & 0xff00) == 0x1000 && (wm == 1 || wm == 2 || wm == 4) &&
