@@ -195,7 +195,8 @@ typedef struct qa_conv_desc {
     int64_t w_code, w_layout, w_kgp, w_rows, wide, needs_rowsum;
     const void* epi_plan;  /* device copy of a qa_plan_epilogue_i8 plan for
                               exactly these parameters, or NULL (MFMA path;
-                              the 128-bit epilogue then runs) */
+                              the 128-bit epilogue then runs); w_code 8: of
+                              the table's qa_plan_lut_i16 plan, or NULL */
     const int64_t* corr;
     const int32_t* boff;
     const int64_t* pre_bias;
@@ -288,6 +289,17 @@ typedef struct qa_epi_params {
 } qa_epi_params;
 int64_t qa_epi_plan_bytes(int64_t cout);
 int qa_plan_epilogue_i8(const qa_epi_params* p, void* plan);
+
+/* Host-side planner of a 16-bit activation table in its LDS form (32 KB for
+ * 65,536 levels): writes a plan of qa_lut_i16_plan_bytes(lut_len) bytes,
+ * whose device copy (16-byte aligned) a w_code 8 descriptor with that table
+ * may carry as epi_plan; its launches then read the table from LDS where
+ * that pays. Returns 1 when planned, 0 when the table is not smooth enough
+ * (entries more than 2 below or 1 above the rounded line between every
+ * 16th in more than two of its groups of 16) or spans more than 65,535, -1 on bad arguments (lut_len 1 to
+ * 65,536). Results do not depend on it. */
+int64_t qa_lut_i16_plan_bytes(int64_t lut_len);
+int qa_plan_lut_i16(const int32_t* lut, int64_t lut_len, void* plan);
 
 /* Float fallbacks on device tensors (the reference's dequantize -> float
  * operator -> quantize, quant_layers.py:195-205), and a strided copy. */

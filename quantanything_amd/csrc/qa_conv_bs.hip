@@ -18,6 +18,12 @@
 // more (the bounds of mul_d), and 4 channels are stored, and their residual
 // read, as 8 bytes. The table reads of all of a lane's values are issued
 // together.
+//
+// YOLOv8n-cls int16, batch 64, 30 launches: 852 -> 500 us in all (stem 80
+// -> 40, 3x3 32 -> 64 at 56x56 35 -> 18, 3x3 256 -> 256 at 7x7 37 -> 14, the
+// 1280 -> 1000 head 31 -> 9). Left: the float64 epilogue, about 100 cycles a
+// value and SIMD, and single waves waiting on their stores between tiles;
+// 16 waves a work-group, or registers held to 4 waves a SIMD, were slower.
 #include <math.h>
 #include <string.h>
 
@@ -44,6 +50,22 @@ struct BsEpi {
 };
 
 constexpr int BIAS_LIM_LOG2 = 51;
+
+// A 16-bit activation table for LDS (qa_plan_lut_i16): {base, entries, two
+// groups}, then per group of 16 consecutive entries 8 bytes: the first entry
+// and the next group's first as uint16 above base, and 2 bits an entry, its
+// difference (+ 2) from the rounded line between them. A smooth table (SiLU
+// over 2^16 levels is within one step of those lines) then takes 32 KB
+// instead of 256 KB; up to two groups that are not (where the clip cuts in)
+// are named in the header, and their entries read from the table itself.
+constexpr int LUTP_HEAD = 16;
+
+__device__ __forceinline__ int lutp_get(const uint2* t, int base, int i) {
+    const uint2 w = t[i >> 4];
+    const int f = i & 15;
+    const int k0 = (int)(w.x & 0xffffu), d = (int)(w.x >> 16) - k0;
+    return base + k0 + ((d * f + 8) >> 4) + (int)(w.y >> (2 * f) & 3u) - 2;
+}
 
 __device__ __noinline__ int bs_exact(const int64_t* pre_p,
                                      const int64_t* mult,
@@ -77,9 +99,14 @@ __device__ __noinline__ int bs_copy_exact(int q, int64_t z, int64_t m,
     return (int)qa_clip128(qa_mbqm_fast((int64_t)q - z, m, sh) + zo, lo, hi);
 }
 
-template <int WM, bool NARROW, bool RES, bool Y2>
+// D: K-steps in flight; a tile's steps are rounded up to whole turns of the
+// ring with steps of zero activations (bs_depth picks D so that there are
+// few), so that every load is unconditional and its wait exact.
+// lutp: the table's LDS form is staged and read (a.plan).
+template <int WM, int D, bool NARROW, bool RES, bool Y2>
 __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
-                                                            BsEpi e) {
+                                                            BsEpi e,
+                                                            int lutp) {
     extern __shared__ int4 bs_dyn[];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15,
               kgl = lane >> 4;
@@ -92,6 +119,7 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
     int8_t* const s_w = (int8_t*)bs_dyn;
     int2* const s_kt = (int2*)(s_w + 2 * WM * nsteps * 1024);
     BsChan* const s_ch = (BsChan*)(s_kt + a.KGp);
+    uint2* const s_lut = (uint2*)(s_ch + 16 * WM);
 
     {   // lane (row col, k-group kgl) of each fragment, straight into LDS
         const int8_t* src = a.ws + (int64_t)g * a.wp_gstride +
@@ -106,6 +134,14 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
                               64 * s;
             __builtin_amdgcn_global_load_lds(p, s_w + 1024 * f, 16, 0, 0);
         }
+    }
+    int4 lhead = int4{0, 0, -1, -1};
+    if (lutp) {
+        const int8_t* src = (const int8_t*)a.plan + LUTP_HEAD;
+        lhead = *(const int4*)a.plan;
+        const int nc = (int)((a.lut_len + 15) / 16 + 1) / 2;  // of 16 bytes
+        for (int c = tid; c < nc; c += 64 * BS_WAVES)
+            ((int4*)s_lut)[c] = ((const int4*)src)[c];
     }
     // the element offset of a k-group's 16 channels from the tap's input
     // pixel (-1: no tap), its displacement dy << 16 | dx
@@ -143,10 +179,8 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
     const int pl = (int)((((uint32_t)pz & 255u) ^ 0x80u) * 0x01010101u);
     const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 
-    // fetch side: (ftile, fs) the next K-step to load
-    constexpr int D = NARROW ? 4 : 3, XW = NARROW ? 1 : 2;
-    int64_t ftile = tile;
-    int fs = 0;
+    constexpr int XW = NARROW ? 1 : 2;
+    const int turns = (nsteps + D - 1) / D * D;
     PixPos fpos = pix_decode(a, tile * 16 + col);
     const int16_t* xb;
     int iy0, ix0, pb;
@@ -160,26 +194,20 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
     origin();
     int4 xr[D][XW];
     bool xin[D];
-    auto fetch = [&](int4 (&x)[XW], bool& in) __attribute__((always_inline)) {
-        if (ftile < ntiles) {
-            const int2 t = s_kt[4 * fs + kgl];
-            in = t.x >= 0 && (unsigned)(iy0 + (t.y >> 16)) < (unsigned)a.H &&
-                 (unsigned)(ix0 + (t.y & 0xffff)) < (unsigned)a.W;
-            // outside: the image's first pixel (in bounds, not used)
-            const int16_t* p = xb + (in ? pb + t.x : 0);
-            if constexpr (NARROW) {
-                const int2 u = *(const int2*)p;
-                x[0] = int4{u.x, u.y, 0, 0};
-            } else {
-                x[0] = *(const int4*)p;
-                x[XW - 1] = *(const int4*)(p + 8);
-            }
-            if (++fs == nsteps) {
-                fs = 0;
-                ftile += tstride;
-                pix_step(a, fpos);
-                origin();
-            }
+    auto fetch = [&](int4 (&x)[XW], bool& in, int s)
+                     __attribute__((always_inline)) {
+        const int2 t = s_kt[4 * min(s, nsteps - 1) + kgl];
+        in = (t.x >= 0) &
+             ((unsigned)(iy0 + (t.y >> 16)) < (unsigned)a.H) &
+             ((unsigned)(ix0 + (t.y & 0xffff)) < (unsigned)a.W);
+        // outside: the image's first pixel (in bounds, not used)
+        const int16_t* p = xb + (in ? pb + t.x : 0);
+        if constexpr (NARROW) {
+            const int2 u = *(const int2*)p;
+            x[0] = int4{u.x, u.y, 0, 0};
+        } else {
+            x[0] = *(const int4*)p;
+            x[XW - 1] = *(const int4*)(p + 8);
         }
     };
     v4i hh[WM], md[WM], ll[WM], sh, sl;
@@ -202,11 +230,14 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
                   (int)__builtin_amdgcn_perm(w.y, w.x, 0x06040200u),
                   (int)__builtin_amdgcn_perm(w.w, w.z, 0x06040200u)};
         xl ^= (int)0x80808080u;
-        if (!in) {
-            xh = v4i{ph, ph, ph, ph};
-            xl = v4i{pl, pl, pl, pl};
+        // (a rounding step's x is 0 in every product and sum)
+        const bool real = s < nsteps;
+        const int vh = real ? ph : 0, vl = real ? pl : 0;
+        if (!(in & real)) {
+            xh = v4i{vh, vh, vh, vh};
+            xl = v4i{vl, vl, vl, vl};
         }
-        const int8_t* f = s_w + 1024 * s + 16 * lane;
+        const int8_t* f = s_w + 1024 * min(s, nsteps - 1) + 16 * lane;
 #pragma unroll
         for (int i = 0; i < WM; ++i) {
             const v4i wh = *(const v4i*)(f + 1024 * i * nsteps);
@@ -272,7 +303,25 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
                         a.qmin, a.qmax);
             }
         }
-        if (a.lut) {  // every table read of the lane in flight
+        if (lutp) {
+            int ix[WM][4];
+            bool odd = false;
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    ix[i][r] = min(max(q[i][r] - loff, 0), lmax);
+                    q[i][r] = lutp_get(s_lut, lhead.x, ix[i][r]);
+                    odd |= (ix[i][r] >> 4) == lhead.z;
+                    odd |= (ix[i][r] >> 4) == lhead.w;
+                }
+            if (__builtin_expect(odd, 0)) {
+#pragma unroll
+                for (int i = 0; i < WM; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) q[i][r] = a.lut[ix[i][r]];
+            }
+        } else if (a.lut) {  // every table read of the lane in flight
 #pragma unroll
             for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -344,26 +393,40 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
             if constexpr (Y2) put((int16_t*)a.y2 + p * a.y2_pst + co, w2);
         }
     };
-    // one copy of the tile's code: the slots move down a step instead of the
-    // loop being unrolled over them
 #pragma unroll
-    for (int d = 0; d < D; ++d) fetch(xr[d], xin[d]);
+    for (int d = 0; d < D; ++d) fetch(xr[d], xin[d], d);
     while (true) {
         clear();
-        for (int cs = 0; cs < nsteps; ++cs) {
-            compute(xr[0], xin[0], cs);
+        int c = 0;
+        for (; c + D < turns; c += D) {
 #pragma unroll
-            for (int d = 0; d + 1 < D; ++d) {
-#pragma unroll
-                for (int k = 0; k < XW; ++k) xr[d][k] = xr[d + 1][k];
-                xin[d] = xin[d + 1];
+            for (int d = 0; d < D; ++d) {
+                compute(xr[d], xin[d], c + d);
+                fetch(xr[d], xin[d], c + d + D);
             }
-            fetch(xr[D - 1], xin[D - 1]);
+        }
+        // the tile's last turn: its slots refill from the wave's next tile
+        // (past the last tile: image 0, in bounds, not used)
+        pix_step(a, fpos);
+        origin();
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            compute(xr[d], xin[d], c + d);
+            fetch(xr[d], xin[d], d);
         }
         finish();
         tile += tstride;
         if (tile >= ntiles) return;
     }
+}
+
+// K-steps in flight: as many as divide the tile's steps, or 3.
+int bs_depth(int nsteps) {
+    return nsteps % 4 == 0 ? 4
+           : nsteps % 3 == 0 ? 3
+           : nsteps <= 2 ? nsteps
+           : nsteps % 2 == 0 && nsteps < 14 ? 2
+                                            : 3;
 }
 
 bool exact_mul(int64_t m, int64_t shift) {  // mul_d's range with tmax 53
@@ -431,7 +494,7 @@ bool launch_conv_bsl(const ConvArgs& b0, bool narrow, int wm,
             wm /= 2;
     }
     while (wm > 1 && bsl_lds(b, wm) > BSL_LDS_MAX) wm /= 2;
-    const int64_t lds = bsl_lds(b, wm);
+    int64_t lds = bsl_lds(b, wm);
     const int64_t gy = ceil_div(b.Cog, 16 * wm);
     BsEpi e;
     memset(&e, 0, sizeof(e));
@@ -456,6 +519,16 @@ bool launch_conv_bsl(const ConvArgs& b0, bool narrow, int wm,
         e.lo2 = (double)b.r2_qmin;
         e.hi2 = (double)b.r2_qmax;
     }
+    // The table's LDS form: a 64-lane read of the 256 KB table takes the
+    // L1 about 64 cycles (a line a lane), its LDS form about 16, for a
+    // staging of up to 32 KB a work-group: worth it past about 4,000 values
+    // a work-group (the YOLOv8n-cls layers up to 14x14).
+    const int64_t nwg = std::min<int64_t>(
+        ceil_div(ntiles, BS_WAVES) * gy * b.G, 2 * (int64_t)cus);
+    const int64_t lutb = round_up(ceil_div(b.lut_len, 16) * 8, 16);
+    const bool lutp = b.lut && b.plan && lds + lutb <= BSL_LDS_MAX &&
+                      b.M * b.Cout >= 4096 * nwg;
+    if (lutp) lds += lutb;
     // (see launch_kernel of the int8 form)
     b.xcd_yfast = 2 * (int64_t)b.N * b.H * b.W * b.Cg * b.G >=
                   2 * (int64_t)b.Cout * b.KGp * 16;
@@ -471,7 +544,7 @@ bool launch_conv_bsl(const ConvArgs& b0, bool narrow, int wm,
         b.st_doy = (int32_t)((stride % ohw) / b.OW);
         b.st_dox = (int32_t)((stride % ohw) % b.OW);
         k<<<dim3((unsigned)gx, (unsigned)gy, (unsigned)b.G), 64 * BS_WAVES,
-            (size_t)lds, st>>>(b, e);
+            (size_t)lds, st>>>(b, e, lutp ? 1 : 0);
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) {
             set_hip_error("k_conv_bsl", err);
@@ -479,22 +552,70 @@ bool launch_conv_bsl(const ConvArgs& b0, bool narrow, int wm,
         }
         return true;
     };
-    auto forms = [&](auto w, auto nr) {
-        constexpr int W = decltype(w)::value;
+    auto forms = [&](auto w, auto dd, auto nr) {
+        constexpr int W = decltype(w)::value, D = decltype(dd)::value;
         constexpr bool NR = decltype(nr)::value;
-        if (b.res && b.y2) return run(&k_conv_bsl<W, NR, true, true>);
-        if (b.res) return run(&k_conv_bsl<W, NR, true, false>);
-        if (b.y2) return run(&k_conv_bsl<W, NR, false, true>);
-        return run(&k_conv_bsl<W, NR, false, false>);
+        if (b.res && b.y2) return run(&k_conv_bsl<W, D, NR, true, true>);
+        if (b.res) return run(&k_conv_bsl<W, D, NR, true, false>);
+        if (b.y2) return run(&k_conv_bsl<W, D, NR, false, true>);
+        return run(&k_conv_bsl<W, D, NR, false, false>);
     };
     using std::integral_constant;
-    if (narrow)
-        return forms(integral_constant<int, 1>{}, std::true_type{});
+    auto depth = [&](auto w, auto nr) {
+        switch (bs_depth(b.KGp / 4)) {
+            case 1: return forms(w, integral_constant<int, 1>{}, nr);
+            case 2: return forms(w, integral_constant<int, 2>{}, nr);
+            case 3: return forms(w, integral_constant<int, 3>{}, nr);
+            default: return forms(w, integral_constant<int, 4>{}, nr);
+        }
+    };
+    if (narrow) return depth(integral_constant<int, 1>{}, std::true_type{});
     switch (wm) {
-        case 1: return forms(integral_constant<int, 1>{}, std::false_type{});
-        case 2: return forms(integral_constant<int, 2>{}, std::false_type{});
-        default: return forms(integral_constant<int, 4>{}, std::false_type{});
+        case 1: return depth(integral_constant<int, 1>{}, std::false_type{});
+        case 2: return depth(integral_constant<int, 2>{}, std::false_type{});
+        default: return depth(integral_constant<int, 4>{}, std::false_type{});
     }
 }
 
 }  // namespace qa
+
+using namespace qa;
+
+QA_API int64_t qa_lut_i16_plan_bytes(int64_t lut_len) {
+    if (lut_len < 1 || lut_len > 65536) return -1;
+    return LUTP_HEAD + round_up(ceil_div(lut_len, 16) * 8, 16);
+}
+
+QA_API int qa_plan_lut_i16(const int32_t* lut, int64_t lut_len, void* plan) {
+    const int64_t bytes = qa_lut_i16_plan_bytes(lut_len);
+    if (!lut || !plan || bytes < 0) return -1;
+    const auto mm = std::minmax_element(lut, lut + lut_len);
+    const int64_t base = *mm.first;
+    if ((int64_t)*mm.second - base > 65535) return 0;
+    memset(plan, 0, (size_t)bytes);
+    int32_t* head = (int32_t*)plan;
+    head[0] = (int32_t)base;
+    head[1] = (int32_t)lut_len;
+    head[2] = head[3] = -1;
+    uint32_t* out = (uint32_t*)((char*)plan + LUTP_HEAD);
+    int odd = 0;
+    for (int64_t i = 0; i < lut_len; i += 16) {
+        const int64_t k0 = lut[i] - base;
+        const int64_t k1 = lut[std::min(i + 16, lut_len - 1)] - base;
+        uint32_t bits = 0;
+        bool fits = true;
+        for (int64_t f = 0; f < 16 && i + f < lut_len; ++f) {
+            const int64_t line = k0 + (((k1 - k0) * f + 8) >> 4);
+            const int64_t r = lut[i + f] - base - line + 2;
+            fits = fits && r >= 0 && r <= 3;
+            bits |= (uint32_t)(r & 3) << (2 * f);
+        }
+        if (!fits) {
+            if (odd == 2) return 0;
+            head[2 + odd++] = (int32_t)(i / 16);
+        }
+        out[i / 8] = (uint32_t)(k0 | k1 << 16);
+        out[i / 8 + 1] = bits;
+    }
+    return 1;
+}

@@ -768,6 +768,7 @@ int desc_args(const qa_conv_desc* d, ConvArgs& a, const char* who) {
         a.wf_rows = (int32_t)rows;
         a.wide = (int32_t)d->wide;
         a.tile_hint = (int32_t)d->tile;
+        a.plan = d->epi_plan;
         if (d->wsplit && d->wsplit_k) {  // the byte-split planes
             int64_t CB, KG, KGp, prow;
             pack_geometry(d->Cout, d->C / d->G, d->KH, d->KW, d->G, 0, &CB,

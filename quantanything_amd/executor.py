@@ -980,6 +980,19 @@ class DeviceExecutor:
                  f"conv:{layer.name}"))
         if d.w_code == 8:
             self.f64_descs.append((d, None, None, f"conv:{layer.name}"))
+            if lut_layer is not None and d.wsplit:
+                p = self._params(lut_layer)
+                if "lut16" not in p:  # the table's LDS form, or None
+                    lut = np.ascontiguousarray(lut_layer.lut, np.int32)
+                    size = self.lib.qa_lut_i16_plan_bytes(len(lut))
+                    plan = np.zeros(max(size, 0), np.uint8)
+                    ok = size > 0 and \
+                        self.lib.qa_plan_lut_i16(
+                            lut.ctypes.data, len(lut),
+                            plan.ctypes.data) == 1
+                    p["lut16"] = _dev(plan, np.uint8) if ok else None
+                if p["lut16"] is not None:
+                    d.epi_plan = p["lut16"].data_ptr()
         name = add_layer or lut_layer or layer
         self.epi[name.node.outputs[0]] = (d, 0, cout)
         self._add(f"conv:{layer.name}", lambda s, d=d:

@@ -87,6 +87,8 @@ def _declare(lib):
         "qa_d_attention": (i32, [p, p]),
         "qa_epi_plan_bytes": (i64, [i64]),
         "qa_plan_epilogue_i8": (i32, [p, p]),
+        "qa_lut_i16_plan_bytes": (i64, [i64]),
+        "qa_plan_lut_i16": (i32, [p, i64, p]),
         "qa_d_requantize": (i32, [p, i32, p, i32] + [i64] * 3 + [p] * 4
                             + [i64] * 5 + [p]),
         "qa_d_rescale": (i32, [p, i32, i64, p, i32] + [i64] * 11 + [p]),

@@ -1,0 +1,65 @@
+"""16-bit convolutions with their weights and activation table in LDS: maps
+large enough that a work-group stages the table, channel counts around the
+16-channel blocks, one to many K-steps (every depth of the ring), a residual
+Add and a Concat copy, inputs past the calibrated range (table clips), all
+against the oracle bit for bit."""
+
+import numpy as np
+import pytest
+
+from oracle.pipeline import OraclePipeline
+from quantanything_amd import graph as G
+from quantanything_amd.container import QuantContainer
+from quantanything_amd.executor import ConvDesc
+from quantanything_amd.synth import Stream
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,cin,cout,k,stride,size,form", [
+    (9, 3, 16, 3, 2, 130, "plain"),     # the 4-channel stem
+    (4, 3, 24, 5, 1, 66, "plain"),      # 25 taps of it: 7 steps
+    (9, 16, 32, 1, 1, 66, "add"),       # one step (of 16 positions)
+    (9, 64, 48, 1, 1, 40, "concat"),    # one step
+    (4, 128, 64, 1, 1, 48, "add"),      # two steps
+    (5, 32, 36, 3, 1, 45, "plain"),     # five steps: rounded up
+    (3, 48, 64, 3, 2, 63, "concat"),    # seven
+    (2, 64, 20, 3, 1, 61, "add"),       # nine
+    (3, 160, 16, 2, 1, 30, "plain"),    # ten
+    (1, 256, 64, 3, 1, 9, "add"),       # 36, few tiles
+])
+def test_bit_exact(hip, tmp_path, n, cin, cout, k, stride, size, form):
+    b = G.GraphBuilder(61)
+    y = b.silu(b.conv("x", cin, cout, k, stride, w_scale=(cin * k * k) ** -.5))
+    if form != "plain":
+        r = b.op("Relu", [b.conv("x", cin, cout, k, stride,
+                                 w_scale=(cin * k * k) ** -.5)])
+        if form == "add":
+            y = b.op("Add", [r, y])
+        else:
+            y = b.op("Concat", [r, y], axis=1)
+    g = b.build("x", [None, cin, size, size], y)
+    shape = (n, cin, size, size)
+    q = QuantContainer(g, "int16", per_channel=True)
+    q.calibrate([Stream(12).normal((1,) + shape[1:]).astype(np.float32)])
+    q.save(tmp_path / "q.json")
+    data = Stream(13).normal(shape, 1.4).astype(np.float32)
+    oracle = OraclePipeline(g, str(tmp_path / "q.json"))
+    oracle.run(data, keep=True)
+    ex = q.executor({"x": shape})
+    ds = [d for d in ex.keep if isinstance(d, ConvDesc)]
+    assert all(d.wsplit for d in ds) and any(d.epi_plan for d in ds)
+    # every channel block: the library's choice, then 1, 2 and 4
+    for code in (0, 0x11011, 0x11012, 0x11014):
+        for d in ds:
+            d.tile = code
+        ex.run({"x": data})
+        checked = 0
+        for name, t in ex.tensors.items():
+            if name in oracle.env:
+                got = t.to_host()
+                np.testing.assert_array_equal(
+                    got, oracle.env[name].reshape(got.shape),
+                    err_msg=f"{name} {code:#x}")
+                checked += 1
+        assert checked >= 1
