@@ -219,7 +219,7 @@ typedef struct qa_conv_desc {
                       work-group split K, lds = weights staged in LDS (a
                       caller's measured choice; ignored where it does not
                       apply); 0x10400: GEMM descriptors (H = W = 1, C a
-                      multiple of 64) on 128 x 128 blocks (0x10403 /
+                      multiple of 16) on 128 x 128 blocks (0x10403 /
                       0x10404: K through 3 / 4 LDS stages filled by direct
                       loads); 0x10800 | wm
                       (wm 1, 2, 4): bands of output rows with the input band
@@ -230,10 +230,9 @@ typedef struct qa_conv_desc {
                       choice) in LDS (layout 0, one group, a table plan,
                       int8 weights without a zero point); 0x12000 |
                       (T - 1) << 4 (T 1..4): 1x1 stride-1 convolutions and
-                      GEMMs of 16, 32 or 64 output channels or a multiple
-                      of 4 above 64 (in blocks of 64), C a multiple of 64
-                      up to 576 (up to 1280 with Cout >= 64 and w_frag), a
-                      table plan without residual (a rescaled copy
+                      GEMMs (in blocks of 64 output channels past 32), C a
+                      multiple of 16 up to 576 (up to 1280 with Cout > 32
+                      and w_frag), a table plan without residual (a rescaled copy
                       allowed): one 16 x 16 block a wave with its weight
                       fragments in registers, T row tiles of 16 a wave, the
                       activation rows staged in LDS (0x12001 is 0x12000).

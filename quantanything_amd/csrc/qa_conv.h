@@ -59,7 +59,8 @@ struct ConvArgs {
     int32_t fastio;                 // y (res, y2): dense channels-last (the
                                     // int8 path: in 4-byte aligned 4-channel
                                     // words)
-    int64_t y_pst, res_pst, y2_pst; // their pixel strides when fastio
+    int32_t rowio;                  // the same at any alignment (word_store)
+    int64_t y_pst, res_pst, y2_pst; // their pixel strides when rowio
     int32_t tile_hint;              // 0, or TILE_VALID | wm | split << 8 |
                                     // lds << 9 (MFMA tile choice)
     int64_t wp_gstride, wp_rstride; // bytes
@@ -200,8 +201,8 @@ bool gemm_big_applies(const ConvArgs& b, int epi);
 // stages 3 or 4: the K loop through that many LDS stages filled by direct
 // loads; otherwise the register-staged two-buffer loop
 bool launch_gemm_big(const ConvArgs& b, hipStream_t st, int stages = 0);
-// Narrow GEMMs / pointwise convolutions (Cout 16, 32, 64 or blocks of 64,
-// K a multiple of 64 up to 576, or 1280 with fragment-order weights, table
+// Narrow GEMMs / pointwise convolutions (up to 16 or 32 channels or blocks of
+// 64, K a multiple of 16 up to 576, or 1280 with fragment-order weights, table
 // plan without residual; a rescaled copy allowed): a 16 x 16 block a wave
 // with its weight fragments in VGPRs (qa_gemm_narrow.hip).
 bool gemm_narrow_applies(const ConvArgs& b, int epi);

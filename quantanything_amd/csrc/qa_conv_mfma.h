@@ -290,6 +290,18 @@ __device__ __forceinline__ int64_t plan_fold(int64_t c, uint32_t corr, int m) {
     return (int64_t)((uint64_t)c + (uint64_t)((int64_t)(int)corr * m));
 }
 
+// A 4-channel word of a row that may start anywhere (the GPU reads and
+// writes unaligned words; rows of a matrix whose width is not a multiple of
+// 4 start off 4 bytes).
+__device__ __forceinline__ uint32_t word_load(const int8_t* p) {
+    uint32_t w;
+    __builtin_memcpy(&w, p, 4);
+    return w;
+}
+__device__ __forceinline__ void word_store(int8_t* p, uint32_t w) {
+    __builtin_memcpy(p, &w, 4);
+}
+
 // Low bytes of four table entries packed into one word (byte = 0), or their
 // second bytes (byte = 1).
 __device__ __forceinline__ uint32_t pack_entries(const int e[4], int byte) {
@@ -513,10 +525,10 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd<WM>(), 8))) void k_conv_mfma(
         for (int i = 0; i < RM; ++i) {
             const int c0 = co0 + i * 16 + cq;
             uint32_t w = 0;
-            if (ok && a.fastio) {
+            if (ok && a.rowio) {
                 const int64_t rb = p * a.res_pst + (int64_t)g * a.Cog + c0;
                 if (c0 + 3 < a.Cog) {
-                    w = *(const uint32_t*)((const int8_t*)a.res + rb);
+                    w = word_load((const int8_t*)a.res + rb);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
@@ -688,7 +700,7 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd<WM>(), 8))) void k_conv_mfma(
                     if (pok) {
                         int8_t* py = (int8_t*)a.y + pq * a.y_pst + cofs;
                         if (c0 + 3 < a.Cog) {
-                            *(uint32_t*)py = wy;
+                            word_store(py, wy);
                         } else {
 #pragma unroll
                             for (int r = 0; r < 4; ++r)
@@ -701,7 +713,7 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd<WM>(), 8))) void k_conv_mfma(
                         if (pok) {
                             int8_t* p2 = (int8_t*)a.y2 + pq * a.y2_pst + cofs;
                             if (c0 + 3 < a.Cog) {
-                                *(uint32_t*)p2 = w2;
+                                word_store(p2, w2);
                             } else {
 #pragma unroll
                                 for (int r = 0; r < 4; ++r)

@@ -10,7 +10,8 @@ bool mfma_launch_lds(const ConvArgs& b, int wm, bool split, int epi,
 }
 
 // The launch form of a descriptor's arguments: whether the output (and
-// residual / copy) is dense channels-last (fastio, pixel strides *_pst),
+// residual / copy) is dense channels-last (rowio; fastio with its words on
+// 4 bytes; pixel strides *_pst),
 // the table epilogue when a plan applies, and the magic divisors of the
 // tap decode. Returns the epilogue variant (epi when no plan applies).
 int fast_io_args(const ConvArgs& a, ConvArgs& b, int epi) {
@@ -22,23 +23,34 @@ int fast_io_args(const ConvArgs& a, ConvArgs& b, int epi) {
         // pixel stride: sp, or the row stride sn of a GEMM (one pixel a row)
         auto pst = [&](int64_t sn, int64_t sp) { return ohw == 1 ? sn : sp; };
         auto dense = [&](const void* p, int64_t sn, int64_t sc, int64_t sp) {
-            return p == nullptr ||
-                   (sc == 1 && (ohw == 1 || sn == ohw * sp) &&
-                    pst(sn, sp) % 4 == 0 && (uintptr_t)p % 4 == 0);
+            return p == nullptr || (sc == 1 && (ohw == 1 || sn == ohw * sp));
         };
-        b.fastio = a.mode == EPI_QUANT &&
-                   (a.G == 1 || a.Cog % 4 == 0 || a.layout == 2) &&
-                   dense(a.y, a.y_sn, a.y_sc, a.y_sp) &&
-                   dense(a.res, a.res_sn, a.res_sc, a.res_sp) &&
-                   dense(a.y2, a.y2_sn, a.y2_sc, a.y2_sp);
+        auto words = [&](const void* p, int64_t sn, int64_t sp) {
+            return p == nullptr ||
+                   (pst(sn, sp) % 4 == 0 && (uintptr_t)p % 4 == 0);
+        };
+        b.rowio = a.mode == EPI_QUANT &&
+                  (a.G == 1 || a.Cog % 4 == 0 || a.layout == 2) &&
+                  dense(a.y, a.y_sn, a.y_sc, a.y_sp) &&
+                  dense(a.res, a.res_sn, a.res_sc, a.res_sp) &&
+                  dense(a.y2, a.y2_sn, a.y2_sc, a.y2_sp);
+        b.fastio = b.rowio && words(a.y, a.y_sn, a.y_sp) &&
+                   words(a.res, a.res_sn, a.res_sp) &&
+                   words(a.y2, a.y2_sn, a.y2_sp);
         b.y_pst = pst(a.y_sn, a.y_sp);
         b.res_pst = pst(a.res_sn, a.res_sp);
         b.y2_pst = pst(a.y2_sn, a.y2_sp);
     }
-    if (a.mode == EPI_QUANT && a.plan && b.fastio) epi = Q8_TABLE;
+    if (a.mode == EPI_QUANT && a.plan && b.rowio) epi = Q8_TABLE;
     b.mg_cb = (((uint64_t)1 << 32) + a.CB - 1) / (uint64_t)a.CB;
     b.mg_kw = (((uint64_t)1 << 32) + a.KW - 1) / (uint64_t)a.KW;
     return epi;
+}
+
+// The 128 x 128 blocks of a GEMM; 0 below 96 columns, which would leave them
+// half empty.
+static int64_t big_blocks(const ConvArgs& b) {
+    return b.Cout < 96 ? 0 : ceil_div(b.M, 128) * ceil_div(b.Cout, 128);
 }
 
 // Tile choice (from measured sweeps over the channel-block width WM and
@@ -55,7 +67,7 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
             return false;
         }
         const int epi = fast_io_args(a, b, Q8_GENERAL);
-        return launch_conv_dw(b, epi, st);
+        return launch_conv_dw(b, b.fastio ? epi : Q8_GENERAL, st);
     }
     if (a.M >= ((int64_t)1 << 31) || a.KGp < 4 || (a.KGp & 3) ||
         a.KGp >= (1 << 16) || a.CB < 1 || a.KW < 1 ||
@@ -98,30 +110,48 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
     if ((a.tile_hint & TILE_VALID) && ((a.tile_hint >> 13) & 1) &&
         gemm_narrow_applies(b, epi))
         return launch_gemm_narrow(b, st, 1 + ((a.tile_hint >> 4) & 3));
-    // large GEMMs: 128 x 128 blocks (tile hint bit 10 chooses; its low
-    // bits 3 or 4 the direct-to-LDS pipeline with that many stages)
-    // (a pointwise convolution over dense pixels is a GEMM of its pixels:
-    // 128 -> 256 channels at 32x56x56 21 us, 33 us on the tiles below;
-    // 384 -> 1280 at 32x14x14 9.9 and 21.3 us)
-    if (b.KH == 1 && b.KW == 1 && b.SH == 1 && b.SW == 1 && b.PH == 0 &&
-        b.PW == 0 && b.OH == b.H && b.OW == b.W &&
-        b.x_sn == (int64_t)b.H * b.W * b.x_sp && b.fastio && b.M > b.N) {
+    // Without a hint (times of a launch in a graph of them, us; blocks =
+    // 16-row x 64-channel blocks):
+    // * a GEMM or pointwise convolution the narrow kernel takes, up to 1024
+    //   blocks (2048 for K of 256 to 576): 4096x576x64 3.8 against 7.1 on the
+    //   tiles below, 197x384x1152 3.6 / 6.4, 1024x1024x1024 7.0 / 9.2 on the
+    //   128 x 128 blocks, which win past it (4096x576x1024 9.9 / 8.2); two
+    //   row tiles a wave past 512 blocks (4096x576x256 5.1 / 5.6); below
+    //   128 channels, where those blocks would be half empty, up to 2048
+    //   (16384x576x64 5.1 / 9.5; 200704x64x32 16.4 against 12.9 on the
+    //   tiles below);
+    // * the 128 x 128 blocks from 32 of them (256x4096x4096: 64 of them,
+    //   25 / 39 us; 1024x4096x256: 16, 24 / 15), K in 64-byte steps through
+    //   three LDS stages (8192x4096x4096 180 against 212 with two register
+    //   buffers, the ViT-S GEMMs 3 - 11% faster). A pointwise convolution
+    //   over dense pixels is a GEMM of its pixels (128 -> 256 channels at
+    //   32x56x56 21 / 33 us, 384 -> 1280 at 32x14x14 9.9 / 21.3).
+    const bool hinted = (a.tile_hint & TILE_VALID) != 0;
+    const bool pointwise = b.KH == 1 && b.KW == 1 && b.SH == 1 &&
+                           b.SW == 1 && b.PH == 0 && b.PW == 0 &&
+                           b.OH == b.H && b.OW == b.W;
+    if (!hinted && pointwise && gemm_narrow_applies(b, epi)) {
+        const int64_t blocks = ceil_div(a.M, 16) * ceil_div(a.Cout, 64);
+        const int K = a.KGp * 16;
+        if (blocks <= 1024 ||
+            (blocks <= 2048 &&
+             (a.Cout < 128 || (K >= 256 && K <= 576))))
+            return launch_gemm_narrow(b, st, blocks > 512 ? 2 : 1);
+    }
+    if (pointwise && b.M > b.N && b.rowio &&
+        b.x_sn == (int64_t)b.H * b.W * b.x_sp) {
         ConvArgs r = b;
         r.N = (int32_t)b.M;
         r.H = r.W = r.OH = r.OW = 1;
         r.x_sn = b.x_sp;
-        if (gemm_big_applies(r, epi) && !(a.tile_hint & TILE_VALID) &&
-            a.M >= 1024 && a.Cout >= 128)
-            return launch_gemm_big(r, st, 0);
+        if (!hinted && gemm_big_applies(r, epi) && big_blocks(r) >= 32)
+            return launch_gemm_big(r, st, 3);
     }
+    // large GEMMs: 128 x 128 blocks (tile hint bit 10 chooses; its low
+    // bits 3 or 4 the direct-to-LDS pipeline with that many stages)
     if (gemm_big_applies(b, epi)) {
-        bool big = a.M >= 1024 && a.Cout >= 128;
-        int stages = 0;
-        if (a.tile_hint & TILE_VALID) {
-            big = (a.tile_hint >> 10) & 1;
-            stages = a.tile_hint & 0xff;
-        }
-        if (big) return launch_gemm_big(b, st, stages);
+        if (hinted ? (a.tile_hint >> 10) & 1 : big_blocks(b) >= 32)
+            return launch_gemm_big(b, st, hinted ? a.tile_hint & 0xff : 3);
     }
     const int64_t ntiles = ceil_div(a.M, 16);
     const int64_t simds = 4 * (int64_t)cu_count();
@@ -135,6 +165,14 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
     int wm = wm_max;
     while (wm > 1 && waves(wm, false) < want) wm >>= 1;
     bool split = a.layout == 0 && KS >= 4 && waves(wm, false) < simds / 2;
+    // up to a wave a SIMD, K split over 32-channel blocks keeps the waves
+    // and halves a wave's steps (64x4096x4096 21.1 -> 14.8 us)
+    // (wave 0 alone finishes a split tile: not with the 128-bit epilogue)
+    if (epi == Q8_TABLE && a.layout == 0 && KS >= 4 && !split && wm == 1 &&
+        a.Cog > 16 && waves(1, false) <= simds) {
+        wm = 2;
+        split = true;
+    }
     // weights staged in LDS when they fit next to the tables (64 KB per
     // work-group), otherwise read from L2
     auto lds_limit = [&](int w) {

@@ -19,7 +19,9 @@
 //
 // Operands: A row p (one pixel of a GEMM descriptor, H = W = 1) at
 // x + p * x_sn, K = Cg bytes; B = the packed weight rows (layout 0, one
-// group), K bytes each, rows padded to 128.
+// group), K bytes each, rows padded to 128. K is Cg rounded up to 64, the
+// weights zero past Cg (a multiple of 16): a 16-byte chunk past the end of an
+// activation row is replaced by the row's first, and left out of its sums.
 #include <type_traits>
 
 #include "qa_conv_mfma.h"
@@ -86,6 +88,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
     const int64_t m0 = (int64_t)(t / nb) * GB_M;
     const int n0 = (t % nb) * GB_N;
     const int K = a.KGp * 16;
+    const int kx = a.Cg;  // bytes of an activation row
     const int nk = K / GB_K;
     const int8_t* xa = (const int8_t*)a.x;
 
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
         for (int j = 0; j < CH; ++j) {
             const int r = lr + j * RSTEP;
             const int4 x = *(const int4*)(xa + min(m0 + r, a.M - 1) * a.x_sn +
-                                          o);
+                                          (o < kx ? o : 0));
             const int4 w =
                 *(const int4*)(a.wp + (int64_t)(n0 + r) * a.wp_rstride + o);
             va[4 * j] = x.x;
@@ -133,17 +136,18 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
     const int lrow = 32 * wave + (lane >> 2);
     const int gch = 16 * ((lane & 3) ^ ((lrow >> 1) & 3));
     const int8_t* const ga0 =
-        xa + min(m0 + lrow, a.M - 1) * a.x_sn + gch;
+        xa + min(m0 + lrow, a.M - 1) * a.x_sn;
     const int8_t* const ga1 =
-        xa + min(m0 + lrow + 16, a.M - 1) * a.x_sn + gch;
+        xa + min(m0 + lrow + 16, a.M - 1) * a.x_sn;
     const int8_t* const gb0 = a.wp + (int64_t)(n0 + lrow) * a.wp_rstride + gch;
     const int8_t* const gb1 = gb0 + 16 * a.wp_rstride;
     // step ks of 64 bytes into stage ks % S (4 direct loads a lane)
     auto dload = [&](int ks) __attribute__((always_inline)) {
         int8_t* const sb = stg + (ks % S) * GB_STAGE + 32 * 64 * wave;
         const int ko = ks * 64;
-        __builtin_amdgcn_global_load_lds(ga0 + ko, sb, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds(ga1 + ko, sb + 16 * 64, 16, 0, 0);
+        const int kc = ko + gch < kx ? ko + gch : 0;
+        __builtin_amdgcn_global_load_lds(ga0 + kc, sb, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(ga1 + kc, sb + 16 * 64, 16, 0, 0);
         __builtin_amdgcn_global_load_lds(gb0 + ko, sb + 8192, 16, 0, 0);
         __builtin_amdgcn_global_load_lds(gb1 + ko, sb + 8192 + 16 * 64, 16,
                                          0, 0);
@@ -199,7 +203,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
         for (int j = 0; j < 4; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     int psum[4] = {0, 0, 0, 0};  // stored-byte sums of the lane's A rows
     // one K-step (BK / 64 MFMA depths) from LDS buffer buf
-    auto mfma_step = [&](int buf) __attribute__((always_inline)) {
+    auto mfma_step = [&](int buf, int ks) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < BK / 64; ++h) {
             v4i fa[4], fb[4];
@@ -217,7 +221,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
                 for (int j = 0; j < 4; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
                         fa[i], fb[j], acc[i][j], 0, 0, 0);
-            if (RS) {
+            if (RS && ks * GB_K + 64 * h + 16 * kg < kx) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) psum[i] += bytes_sum(fa[i], 16);
             }
@@ -227,7 +231,8 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
     // kg ^ ((col >> 1) & 3) of the row (the tile's row bases are multiples
     // of 16)
     const int foff = col * 64 + 16 * (kg ^ ((col >> 1) & 3));
-    auto mfma_stage = [&](const int8_t* sb) __attribute__((always_inline)) {
+    auto mfma_stage = [&](const int8_t* sb, int ks)
+                          __attribute__((always_inline)) {
         v4i fa[4], fb[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -241,7 +246,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
             for (int j = 0; j < 4; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
                     fa[i], fb[j], acc[i][j], 0, 0, 0);
-        if (RS) {
+        if (RS && 64 * ks + 16 * kg < kx) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) psum[i] += bytes_sum(fa[i], 16);
         }
@@ -261,7 +266,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             if (ks + S - 1 < nk) dload(ks + S - 1);
-            mfma_stage(stg + (ks % S) * GB_STAGE);
+            mfma_stage(stg + (ks % S) * GB_STAGE, ks);
         }
 #pragma unroll
         for (int j = 0; j < 3; ++j) s_tab[tid + 256 * j] = tv[j];
@@ -278,7 +283,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
                 sstore(ra[sl], rb[sl], ks & 1);
                 if (ks + P < nk) gload(ra[sl], rb[sl], ks + P);
                 __syncthreads();
-                mfma_step(ks & 1);
+                mfma_step(ks & 1, ks);
             }
         }
     }
@@ -325,10 +330,10 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
                     const int8_t* pr =
                         (const int8_t*)a.res + pq * a.res_pst + c0;
                     if (!CHK) {
-                        w = *(const uint32_t*)pr;
+                        w = word_load(pr);
                     } else if (pok) {
                         if (cfull) {
-                            w = *(const uint32_t*)pr;
+                            w = word_load(pr);
                         } else {
 #pragma unroll
                             for (int r = 0; r < 4; ++r)
@@ -363,8 +368,8 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
                 int8_t* p2 = Y2 ? (int8_t*)a.y2 + pq * a.y2_pst + c0
                                 : nullptr;
                 if (!CHK || (pok && cfull)) {
-                    *(uint32_t*)py = wy;
-                    if (Y2) *(uint32_t*)p2 = w2;
+                    word_store(py, wy);
+                    if (Y2) word_store(p2, w2);
                 } else if (pok) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
@@ -392,11 +397,11 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
 
 bool gemm_big_applies(const ConvArgs& b, int epi) {
     const uintptr_t xa = (uintptr_t)b.x;
-    return epi == Q8_TABLE && b.mode == EPI_QUANT && b.fastio && b.plan &&
+    return epi == Q8_TABLE && b.mode == EPI_QUANT && b.rowio && b.plan &&
            b.G == 1 && b.layout == 0 && b.KH == 1 && b.KW == 1 &&
            b.H == 1 && b.W == 1 && b.OH == 1 && b.OW == 1 && b.x_code == 1 &&
-           b.x_sc == 1 && b.Cg % 64 == 0 && b.Cg <= 16384 &&
-           b.KGp * 16 == b.Cg &&
+           b.x_sc == 1 && b.Cg % 16 == 0 && b.Cg <= 16384 &&
+           b.KGp * 16 == round_up(b.Cg, 64) &&
            b.wp_rstride == (int64_t)b.KGp * 16 && b.x_sn % 16 == 0 &&
            xa % 16 == 0 && b.y_code == 1 && b.M < ((int64_t)1 << 31);
 }

@@ -1,7 +1,8 @@
 // Narrow int8 GEMMs and pointwise convolutions with the table epilogue:
-// 16, 32 or 64 output channels, or any multiple of 4 in blocks of 64; K a
-// multiple of 64 up to 576 (1280 in 64-channel blocks with the weights in
-// fragment order); any number of rows M (the standalone 4096 x 576 x 64
+// up to 16 or 32 output channels, or any number in blocks of 64; K a
+// multiple of 16 up to 576 (1280 in 64-channel blocks with the weights in
+// fragment order), its last 64-byte step's missing chunks standing against
+// zero weights; output rows at any alignment; any number of rows M (the standalone 4096 x 576 x 64
 // GEMM, the 1x1 convolutions of a classifier's late stages, its
 // 1280 -> 1000 head).
 //
@@ -54,7 +55,7 @@ struct GnArgs {
     int8_t* y;             // output rows, ypst bytes apart
     int8_t* y2;            // the rescaled copy (NULL: none), y2pst apart
     int64_t xpst, ypst, y2pst, M;
-    int32_t KGp, Cout, RTL, pad;
+    int32_t KGp, Cout, RTL, kx;  // kx: bytes of an activation row
     // CV (a k x k convolution, Cg a multiple of 64): the image geometry;
     // row p is output pixel p of the batch, K-step s covers tap s / CBK,
     // input channels 64 (s % CBK) ..; x_sn / xpst: image / pixel strides
@@ -77,11 +78,11 @@ struct GnArgs {
 // GEMM row's); a tap outside the image loads pixel (0, 0) and then has
 // its LDS bytes overwritten with the pad value.
 #define GN_ARGS(g) \
-    (g).x, (g).wf, (g).plan, (g).xpst, (g).M, (g).KGp, (g).RTL, (g)
+    (g).x, (g).wf, (g).plan, (g).xpst, (g).M, (g).KGp, (g).RTL, (g).kx, (g)
 template <int NB, bool RS, bool WF, int KM, bool CV = false>
 __global__ __launch_bounds__(256) void k_gemm_narrow(
     const int8_t* x, const int8_t* wf, const char* plan, int64_t xpst,
-    int64_t M, int32_t KGp, int32_t RTL, GnArgs a) {
+    int64_t M, int32_t KGp, int32_t RTL, int32_t kx, GnArgs a) {
     constexpr int RT = 4 / NB;
     constexpr int RW = 16 * NB;  // weight rows
     extern __shared__ int4 gn_dyn[];
@@ -103,15 +104,16 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
     // position l % 4), then the constants
     const int tv = ((const int*)(plan + PLAN_E))[tid];
     const int g = lane >> 2, q = lane & 3;
+    // (a chunk past the row's bytes: its first one, against zero weights)
     auto dloads = [&](const int8_t* base, int64_t rs, int R, int64_t rmax,
-                      int8_t* dst) __attribute__((always_inline)) {
+                      int8_t* dst, int bytes) __attribute__((always_inline)) {
         const int n = R * nks / 16;  // instructions (R a multiple of 16)
         for (int i = wave; i < n; i += 4) {
             const int sg = 16 * i + g, st = sg / R, r = sg - st * R;
             const int64_t row = min((int64_t)r, rmax);
+            const int o = 64 * st + 16 * (q ^ ((r >> 2) & 3));
             __builtin_amdgcn_global_load_lds(
-                base + row * rs + 64 * st + 16 * (q ^ ((r >> 2) & 3)),
-                dst + 1024 * i, 16, 0, 0);
+                base + row * rs + (o < bytes ? o : 0), dst + 1024 * i, 16, 0, 0);
         }
     };
     v4i fwr[KM];
@@ -145,10 +147,11 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
                 s_x + 1024 * i, 16, 0, 0);
         }
     } else {
-        dloads(x + px * xpst, xpst, RX, M - 1 - px, s_x);
+        dloads(x + px * xpst, xpst, RX, M - 1 - px, s_x, kx);
     }
     if (!WF)  // weight rows cw .. cw + RW - 1 (packed rows padded to 128)
-        dloads(a.wp + (int64_t)cw * 16 * KGp, 16 * KGp, RW, RW - 1, s_w);
+        dloads(a.wp + (int64_t)cw * 16 * KGp, 16 * KGp, RW, RW - 1, s_w,
+               16 * KGp);
     const int4 hdr = *(const int4*)plan;
     const int pD = ((const int*)plan)[4];
     int4 pc[4];
@@ -190,7 +193,7 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
                           crr[r], pc[r].x);
     const int pA = hdr.x, pB = hdr.y;
     const bool idt = hdr.w & PLAN_IDENT;
-    const int cs = c0 + 4 * kg;  // the lane's 4 channels (Cout % 4 == 0)
+    const int cs = c0 + 4 * kg;  // the lane's 4 channels
     // row tile j = wave / NB + RT t of the work-group: rows 16 j + col,
     // chunk kg of K-step s
     for (int t = 0; t < RTL; ++t) {
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
                 const v4i fx = *(const v4i*)(fx0 + s * RX * 64);
                 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fwr[s], fx, acc,
                                                            0, 0, 0);
-                if (RS) psum += bytes_sum(fx, 16);
+                if (RS && 64 * s + 16 * kg < kx) psum += bytes_sum(fx, 16);
             }
         }
         if (RS) {  // the row's byte sum over its 4 k-group lanes
@@ -223,9 +226,18 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
         }
         const int64_t p = px + 16 * j + col;
         if (p < M && cs < a.Cout) {
-            *(uint32_t*)(a.y + p * a.ypst + cs) = pack_entries(e, 0);
-            if (a.y2)
-                *(uint32_t*)(a.y2 + p * a.y2pst + cs) = pack_entries(e, 1);
+            auto put = [&](int8_t* d, uint32_t w)
+                           __attribute__((always_inline)) {
+                if (cs + 3 < a.Cout) {
+                    word_store(d, w);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 3; ++r)
+                        if (cs + r < a.Cout) d[r] = (int8_t)(w >> (8 * r));
+                }
+            };
+            put(a.y + p * a.ypst + cs, pack_entries(e, 0));
+            if (a.y2) put(a.y2 + p * a.y2pst + cs, pack_entries(e, 1));
         }
     }
 }
@@ -236,16 +248,15 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
 // (tile codes with the weights in fragment order).
 bool narrow_conv_applies(const ConvArgs& b, int epi) {
     const uintptr_t xa = (uintptr_t)b.x;
-    return epi == Q8_TABLE && b.mode == EPI_QUANT && b.fastio && b.plan &&
+    return epi == Q8_TABLE && b.mode == EPI_QUANT && b.rowio && b.plan &&
            !b.res && b.G == 1 && b.layout == 0 && b.wfrag &&
            (b.KH > 1 || b.KW > 1 || b.SH > 1 || b.SW > 1 || b.PH > 0 ||
             b.PW > 0 || b.OH != b.H || b.OW != b.W) &&
            b.x_code == 1 && b.x_sc == 1 && b.Cg % 64 == 0 &&
            b.x_sp % 16 == 0 && b.x_sn % 16 == 0 && xa % 16 == 0 &&
            b.KGp * 16 == b.Cg * b.KH * b.KW &&
-           b.Cout >= 16 && b.Cout % 4 == 0 &&
-           (b.Cout <= 64 ? b.Cout % 16 == 0 : b.Cout <= 64 * 65535) &&
-           (b.KGp <= 36 || (b.KGp <= 4 * GN_KMAX && b.Cout >= 64)) &&
+           b.Cout <= 64 * 65535 &&
+           (b.KGp <= 36 || (b.KGp <= 4 * GN_KMAX && b.Cout > 32)) &&
            b.wp_rstride == (int64_t)b.KGp * 16 && b.y_code == 1 &&
            b.M < ((int64_t)1 << 31) &&
            (int64_t)b.OH * b.OW < ((int64_t)1 << 31) &&
@@ -259,23 +270,22 @@ bool gemm_narrow_applies(const ConvArgs& b, int epi) {
     // a row's stride: the GEMM's row stride, or the pixel stride of a
     // dense channels-last tensor
     const int64_t xpst = hw == 1 ? b.x_sn : b.x_sp;
-    return epi == Q8_TABLE && b.mode == EPI_QUANT && b.fastio && b.plan &&
+    return epi == Q8_TABLE && b.mode == EPI_QUANT && b.rowio && b.plan &&
            !b.res && b.G == 1 && b.layout == 0 && b.KH == 1 &&
            b.KW == 1 && b.SH == 1 && b.SW == 1 && b.PH == 0 && b.PW == 0 &&
            b.OH == b.H && b.OW == b.W && (hw == 1 || b.x_sn == hw * b.x_sp) &&
            b.x_code == 1 && b.x_sc == 1 && xpst % 16 == 0 && xa % 16 == 0 &&
-           b.Cout >= 16 && b.Cout % 4 == 0 &&
-           (b.Cout <= 64 ? b.Cout % 16 == 0 : b.Cout <= 64 * 65535) &&
-           b.Cg % 64 == 0 && b.KGp * 16 == b.Cg &&
+           b.Cout <= 64 * 65535 &&
+           b.Cg % 16 == 0 && b.KGp * 16 == round_up(b.Cg, 64) &&
            (b.KGp <= 36 ||
-            (b.KGp <= 4 * GN_KMAX && b.Cout >= 64 && b.wfrag)) &&
+            (b.KGp <= 4 * GN_KMAX && b.Cout > 32 && b.wfrag)) &&
            b.wp_rstride == (int64_t)b.KGp * 16 && b.y_code == 1 &&
            b.M < ((int64_t)1 << 31);
 }
 
 bool launch_gemm_narrow(const ConvArgs& b, hipStream_t st, int rtl) {
-    // Cout 16 / 32 / 64: one channel block of Cout; beyond, blocks of 64
-    const int nb = b.Cout <= 64 ? b.Cout / 16 : 4;
+    // up to 16 / 32 channels: one block of that many; beyond, blocks of 64
+    const int nb = b.Cout <= 16 ? 1 : b.Cout <= 32 ? 2 : 4;
     // row tiles a wave: 1..4, fewer where the rows would not fit in 64 KB
     // of LDS (results do not depend on it)
     const int64_t per = (int64_t)(b.KGp / 4) * 64 * 16 * (4 / nb);
@@ -305,8 +315,8 @@ bool launch_gemm_narrow(const ConvArgs& b, hipStream_t st, int rtl) {
     g.KGp = b.KGp;
     g.Cout = b.Cout;
     g.RTL = rtl;
-    g.pad = 0;
     const bool cv = narrow_conv_applies(b, Q8_TABLE);
+    g.kx = cv ? b.KGp * 16 : b.Cg;
     if (cv) {
         g.xpst = b.x_sp;
         g.x_sn = b.x_sn;

@@ -2266,9 +2266,9 @@ class DeviceExecutor:
         convolution or GEMM, or a k x k convolution as a GEMM over its
         im2col rows)."""
         k = d.C * d.KH * d.KW  # K of the GEMM (of the im2col rows)
-        return d.G == 1 and d.w_layout == 0 and d.Cout >= 16 and \
-            d.Cout % 4 == 0 and (d.Cout > 64 or d.Cout % 16 == 0) and \
-            d.C % 64 == 0 and (k <= 576 or (k <= 1280 and d.Cout >= 64)) \
+        return d.G == 1 and d.w_layout == 0 and d.w_code == 1 and \
+            d.C % (16 if d.KH == d.KW == 1 else 64) == 0 and \
+            (k <= 576 or (k <= 1280 and d.Cout > 32)) \
             and bool(d.epi_plan) and not d.res
 
     @staticmethod
@@ -2295,7 +2295,7 @@ class DeviceExecutor:
         wm_max = 1 if cog <= 16 else 2 if cog <= 32 else 4 if cog <= 64 else 8
         out = [0]
         if d.H == d.W == d.KH == d.KW == 1 and d.G == 1 and \
-                d.w_layout == 0 and d.C % 64 == 0:
+                d.w_layout == 0 and d.C % 16 == 0:
             # the large-GEMM kernel (128 x 128 blocks): K steps staged
             # through registers, or through 3 / 4 LDS stages of direct loads
             out += [0x10400, 0x10403, 0x10404]

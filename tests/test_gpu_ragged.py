@@ -85,3 +85,36 @@ def test_other_readers_see_the_rows(hip, tmp_path):
     y = b.op("Concat", [h, z], axis=1)
     _check(b.build("x", [None, 30], [y, z]), "int8", (19, 30), tmp_path,
            rows=64)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1, 16, 1), (19, 48, 5), (130, 80, 17), (300, 208, 33), (77, 592, 65),
+    (260, 1040, 131), (1030, 144, 250), (64, 1264, 37), (515, 2064, 258)])
+def test_gemm_rows_off_the_grid(hip, m, k, n):
+    """Every kernel a GEMM descriptor can take, K a multiple of 16 alone and
+    output rows of any width, against 64-bit integers; the bytes after the
+    output stay."""
+    import torch
+
+    from quantanything_amd.executor import DeviceExecutor
+    from quantanything_amd.workloads import GemmWorkload
+
+    w = GemmWorkload(seed=m + n, M=m, K=k, N=n)
+    w.y = torch.full((m * n + 64,), 77, dtype=torch.int8, device="cuda")
+    w.d.y = w.y.data_ptr()
+    g = w.spec
+    acc = (g["a"].astype(np.int64) - g["zp_in"]) @ g["w"].astype(np.int64)
+    t = 31 + g["shift"]
+    q = ((acc + g["bias"]) * g["mult"] + (1 << (t - 1))) >> t
+    want = (np.clip(q + g["zp_out"], g["qmin"], g["qmax"]) - 128)
+    codes = DeviceExecutor.tile_candidates(w.d)
+    assert any(c >> 13 & 1 for c in codes) == (k <= 576 or
+                                              (k <= 1280 and n > 32))
+    for code in codes + [0x10400, 0x10403, 0x10404]:
+        w.d.tile = code
+        w.y.fill_(77)
+        w.launch()
+        got = w.y.cpu().numpy()
+        np.testing.assert_array_equal(got[:m * n].reshape(m, n), want,
+                                      err_msg=hex(code))
+        assert (got[m * n:] == 77).all(), hex(code)
