@@ -105,7 +105,7 @@ __global__ __launch_bounds__(WR_NT) void k_conv_wr(ConvArgs a, WrGeom bg,
     const XcdBlock blk = xcd_block(true);
     const int co0 = (int)blk.y * WM * 16;
     const int KGp = a.KGp;
-    const int cpp = a.Cg >> 4;  // 16-byte chunks per input pixel
+    const int cpp = a.CB;  // 16-byte chunks per input pixel
     const int nch = bg.BR * bg.BW * cpp;
     const int pv = splat4(a.pad_value);
     const v4i pad4 = {pv, pv, pv, pv};
@@ -564,14 +564,14 @@ WrGeom wr_geom(const ConvArgs& b, int wm, int R, bool ch = false) {
     g.R = R;
     g.BR = (R - 1) * b.SH + (b.KH - 1) * b.DH + 1;
     g.BW = (b.OW - 1) * b.SW + (b.KW - 1) * b.DW + 1;
-    g.PS = b.Cg + (((b.Cg >> 4) & 1) ? 0 : 16);
+    g.PS = 16 * b.CB + ((b.CB & 1) ? 0 : 16);
     g.bpi = (b.OH + R - 1) / R;
     g.nbands = b.N * g.bpi;
     g.KSR = wr_steps(wm, b.KGp / 4);
     // weight rows hold the instantiated K-steps (the tail chunks zeroed)
     g.RSW = std::max<int>(4 * g.KSR, b.KGp) * 16 + 16;
     const int64_t band = (int64_t)g.BR * g.BW * g.PS;
-    const int64_t bchunks = (int64_t)g.BR * b.W * (b.Cg >> 4);
+    const int64_t bchunks = (int64_t)g.BR * b.W * b.CB;
     const int64_t wchunks = (int64_t)wm * 16 * b.KGp;
     g.band_bytes = (int)std::min<int64_t>(band, 1 << 30);
     auto magic = [](int64_t d) {
@@ -582,7 +582,7 @@ WrGeom wr_geom(const ConvArgs& b, int wm, int R, bool ch = false) {
     g.m_kgp = magic(b.KGp);
     g.m_ow = magic(b.OW);
     g.m_w = magic(b.W);
-    g.m_cpp = magic(b.Cg >> 4);
+    g.m_cpp = magic(b.CB);
     int64_t bytes =
         band + (int64_t)wm * 16 * g.RSW + (int64_t)g.KSR * 16 +
         (ch ? (int64_t)wm * 16 * 80 + WR_NW * 16 * 80 : 0);
@@ -600,7 +600,7 @@ WrGeom wr_geom(const ConvArgs& b, int wm, int R, bool ch = false) {
     // gfx950 gives a work-group up to 160 KB of LDS
     g.lds = bytes <= 150 * 1024 && bchunks <= (int64_t)WR_SB * WR_NT &&
                     wchunks <= (int64_t)WR_SW * WR_NT &&
-                    (int64_t)g.BR * g.BW * (b.Cg >> 4) < (1 << 16)
+                    (int64_t)g.BR * g.BW * b.CB < (1 << 16)
                 ? (int)bytes
                 : 0;
     return g;
@@ -656,7 +656,8 @@ bool conv_wr_applies(const ConvArgs& b, int epi, int wm) {
     if (wm != 1 && wm != 2 && wm != 4) return false;
     if (!(epi == Q8_TABLE && b.mode == EPI_QUANT && b.fastio && b.plan &&
           b.G == 1 && b.layout == 0 && b.x_code == 1 && b.x_sc == 1 &&
-          b.rowsum == 0 && b.Cg % 16 == 0 && b.Cg > 0 &&
+          // (a pixel's last 16 bytes may pass its channels: zero weights)
+          b.rowsum == 0 && b.Cg > 0 && b.x_sp >= 16 * (int64_t)b.CB &&
           b.W >= 2 &&
           b.Cout % 4 == 0 &&
           b.OW >= 2 &&
