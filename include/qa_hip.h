@@ -219,9 +219,11 @@ typedef struct qa_conv_desc {
                       work-group split K, lds = weights staged in LDS (a
                       caller's measured choice; ignored where it does not
                       apply); 0x10400: GEMM descriptors (H = W = 1, C a
-                      multiple of 16) on 128 x 128 blocks (0x10403 /
-                      0x10404: K through 3 / 4 LDS stages filled by direct
-                      loads); 0x10800 | wm
+                      multiple of 16) on large blocks, K through LDS
+                      stages filled by direct loads (the library's choice of
+                      block; 0x10403 / 0x10404: 128 x 128 with 3 / 4 stages,
+                      0x10410: 64 x 128, 0x10411: 256 x 256, 0x10412:
+                      256 x 128); 0x10800 | wm
                       (wm 1, 2, 4): bands of output rows with the input band
                       and the weights in LDS (layout 0, one group, a table
                       plan); 0x11000 | wm | R << 4 (wm 1, 2, 4): the weights

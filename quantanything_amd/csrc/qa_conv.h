@@ -194,13 +194,13 @@ bool launch_conv_valu(const ConvArgs& a, hipStream_t st);
 // form, `epi` as chosen by launch_conv_mfma.
 bool conv_dw_applies(const ConvArgs& b);
 bool launch_conv_dw(const ConvArgs& b, int epi, hipStream_t st);
-// Large GEMM descriptors (H = W = 1, K a multiple of 64) with the int8 table
-// epilogue on 128 x 128 blocks (qa_gemm_big.hip); `epi` as chosen by
-// launch_conv_mfma.
+// Large GEMM descriptors (H = W = 1, C a multiple of 16) with the int8 table
+// epilogue; `epi` as chosen by launch_conv_mfma.
 bool gemm_big_applies(const ConvArgs& b, int epi);
-// stages 3 or 4: the K loop through that many LDS stages filled by direct
-// loads; otherwise the register-staged two-buffer loop
-bool launch_gemm_big(const ConvArgs& b, hipStream_t st, int stages = 0);
+// on 128 x 128 blocks, K through 3 or 4 LDS stages (qa_gemm_big.hip)
+bool launch_gemm_big(const ConvArgs& b, hipStream_t st, int stages);
+// on the blocks `form` names, 0: chosen by size (qa_gemm_stage.hip)
+bool launch_gemm_stage(const ConvArgs& b, hipStream_t st, int form);
 // Narrow GEMMs / pointwise convolutions (up to 16 or 32 channels or blocks of
 // 64, K a multiple of 16 up to 576, or 1280 with fragment-order weights, table
 // plan without residual; a rescaled copy allowed): a 16 x 16 block a wave

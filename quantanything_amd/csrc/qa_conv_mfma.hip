@@ -114,18 +114,17 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
     // 16-row x 64-channel blocks):
     // * a GEMM or pointwise convolution the narrow kernel takes, up to 1024
     //   blocks (2048 for K of 256 to 576): 4096x576x64 3.8 against 7.1 on the
-    //   tiles below, 197x384x1152 3.6 / 6.4, 1024x1024x1024 7.0 / 9.2 on the
-    //   128 x 128 blocks, which win past it (4096x576x1024 9.9 / 8.2); two
+    //   tiles below, 197x384x1152 3.6 / 6.4, 1024x1024x1024 6.6 / 6.5 on the
+    //   staged blocks, which win past it (4096x576x1024 9.9 / 8.2); two
     //   row tiles a wave past 512 blocks (4096x576x256 5.1 / 5.6); below
     //   128 channels, where those blocks would be half empty, up to 2048
     //   (16384x576x64 5.1 / 9.5; 200704x64x32 16.4 against 12.9 on the
     //   tiles below);
-    // * the 128 x 128 blocks from 32 of them (256x4096x4096: 64 of them,
-    //   25 / 39 us; 1024x4096x256: 16, 24 / 15), K in 64-byte steps through
-    //   three LDS stages (8192x4096x4096 180 against 212 with two register
-    //   buffers, the ViT-S GEMMs 3 - 11% faster). A pointwise convolution
-    //   over dense pixels is a GEMM of its pixels (128 -> 256 channels at
-    //   32x56x56 21 / 33 us, 384 -> 1280 at 32x14x14 9.9 / 21.3).
+    // * the staged blocks of launch_gemm_stage from 16 blocks of 128 x 128
+    //   (1024x4096x256, 16 of them: 13.0 us against 14.5 on the tiles below;
+    //   256x4096x4096, 64: 16.7 / 39). A pointwise convolution over dense
+    //   pixels is a GEMM of its pixels (128 -> 256 channels at 32x56x56
+    //   21 / 33 us, 384 -> 1280 at 32x14x14 9.9 / 21.3).
     const bool hinted = (a.tile_hint & TILE_VALID) != 0;
     const bool pointwise = b.KH == 1 && b.KW == 1 && b.SH == 1 &&
                            b.SW == 1 && b.PH == 0 && b.PW == 0 &&
@@ -144,14 +143,13 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
         r.N = (int32_t)b.M;
         r.H = r.W = r.OH = r.OW = 1;
         r.x_sn = b.x_sp;
-        if (!hinted && gemm_big_applies(r, epi) && big_blocks(r) >= 32)
-            return launch_gemm_big(r, st, 3);
+        if (!hinted && gemm_big_applies(r, epi) && big_blocks(r) >= 16)
+            return launch_gemm_stage(r, st, 0);
     }
-    // large GEMMs: 128 x 128 blocks (tile hint bit 10 chooses; its low
-    // bits 3 or 4 the direct-to-LDS pipeline with that many stages)
+    // large GEMMs (tile hint bit 10 chooses them, its low byte the blocks)
     if (gemm_big_applies(b, epi)) {
-        if (hinted ? (a.tile_hint >> 10) & 1 : big_blocks(b) >= 32)
-            return launch_gemm_big(b, st, hinted ? a.tile_hint & 0xff : 3);
+        if (hinted ? (a.tile_hint >> 10) & 1 : big_blocks(b) >= 16)
+            return launch_gemm_stage(b, st, hinted ? a.tile_hint & 0xff : 0);
     }
     const int64_t ntiles = ceil_div(a.M, 16);
     const int64_t simds = 4 * (int64_t)cu_count();

@@ -6,11 +6,10 @@
 // matrix cores waiting on the memory pipe. Here a work-group computes a
 // 128 x 128 block of C: its 4 waves (2 x 2) own 64 x 64 each, i.e. 4 x 4
 // MFMA tiles of v_mfma_i32_16x16x64_i8, so every A fragment feeds 4 MFMAs
-// and every B fragment 4. K runs in 64- or 128-byte steps through two LDS
-// buffers (global -> registers for the next step while a step's MFMAs run,
-// one barrier a step), or (S > 0) in 64-byte steps through S LDS stages
-// filled straight from global memory (global_load_lds_dwordx4: no
-// registers hold loads in flight, so S - 1 steps are requested ahead). The epilogue is the int8 table plan of qa_conv.h
+// and every B fragment 4. K runs in 64-byte steps
+// through S LDS stages filled straight from global memory
+// (global_load_lds_dwordx4: no registers hold loads in flight, so S - 1
+// steps are requested ahead). The epilogue is the int8 table plan of qa_conv.h
 // (per-channel multiply-add and shift, 256-entry clip / activation /
 // residual / copy tables), identical in results to the convolution
 // kernel's; residual, copy and pixel sums are template flags, full tiles
@@ -31,14 +30,9 @@ namespace {
 
 constexpr int GB_M = 128, GB_N = 128;
 
-// BK: K bytes a step (64 or 128: one or two MFMA K-depths per barrier);
-// P: steps whose global loads are in flight (a ring of P register slots:
-// step k's operands are requested when step k - P is stored to LDS, so the
-// memory latency is covered by P steps of MFMAs; with K <= P * BK every
-// load is issued before the first MFMA).
 // RES / Y2 / RS: residual Add, rescaled second output, pixel sums of the
 // activations (weights with an offset) in the epilogue.
-// S > 0 (BK 64, P unused): stage s holds A (128 rows x 64 bytes) and B
+// Stage s holds A (128 rows x 64 bytes) and B
 // (128 x 64) at dynamic LDS bytes 16384 s and 16384 s + 8192; row r's
 // 16-byte chunk c sits at position c ^ ((r >> 1) & 3) of the row, so that
 // the 8 rows one fragment read serves at a time fall in distinct banks
@@ -55,17 +49,9 @@ __device__ __forceinline__ void wait_vm(int n) {
         default: __builtin_amdgcn_s_waitcnt(0x0f7c); break;
     }
 }
-template <int P, int BK, bool RES, bool Y2, bool RS, int S>
+template <bool RES, bool Y2, bool RS, int S>
 __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
-    static_assert(S == 0 || (BK == 64 && S >= 2 && S <= 5), "stages");
-    constexpr int GB_K = BK;
-    constexpr int GB_RS = BK + 16;  // LDS row stride (bytes)
-    constexpr int CPR = BK / 16;    // 16-byte chunks per row
-    constexpr int CH = GB_M * CPR / 256;  // chunks per thread and operand
-    // the two register-path buffers (S > 0: the dynamic stages instead)
-    constexpr int SAB = S > 0 ? 16 : GB_M * GB_RS;
-    __shared__ __attribute__((aligned(16))) int8_t sA[2][SAB];
-    __shared__ __attribute__((aligned(16))) int8_t sB[2][SAB];
+    static_assert(S >= 2 && S <= 5, "stages");
     extern __shared__ int4 gb_dyn[];
     __shared__ int s_tab[768];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -89,48 +75,10 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
     const int n0 = (t % nb) * GB_N;
     const int K = a.KGp * 16;
     const int kx = a.Cg;  // bytes of an activation row
-    const int nk = K / GB_K;
+    const int nk = K / 64;
     const int8_t* xa = (const int8_t*)a.x;
 
-    // global -> registers: per operand and step, CH chunks of 16 bytes per
-    // thread (chunk tid + 256 j: row (tid / CPR) + j * 256 / CPR, bytes
-    // 16 (tid % CPR)); loads past the last step re-read it (in bounds,
-    // unused)
-    constexpr int RSTEP = 256 / CPR;  // rows between a thread's chunks
-    const int lr = tid / CPR, lk = (tid % CPR) * 16;
-    typedef int vch __attribute__((ext_vector_type(4 * CH)));
-    vch ra[S > 0 ? 1 : P], rb[S > 0 ? 1 : P];
-    auto gload = [&](vch& va, vch& vb, int ks) __attribute__((always_inline)) {
-        const int o = min(ks, nk - 1) * GB_K + lk;
-#pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const int r = lr + j * RSTEP;
-            const int4 x = *(const int4*)(xa + min(m0 + r, a.M - 1) * a.x_sn +
-                                          (o < kx ? o : 0));
-            const int4 w =
-                *(const int4*)(a.wp + (int64_t)(n0 + r) * a.wp_rstride + o);
-            va[4 * j] = x.x;
-            va[4 * j + 1] = x.y;
-            va[4 * j + 2] = x.z;
-            va[4 * j + 3] = x.w;
-            vb[4 * j] = w.x;
-            vb[4 * j + 1] = w.y;
-            vb[4 * j + 2] = w.z;
-            vb[4 * j + 3] = w.w;
-        }
-    };
-    auto sstore = [&](const vch& va, const vch& vb, int buf)
-                      __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const int r = lr + j * RSTEP;
-            *(int4*)&sA[buf][r * GB_RS + lk] =
-                int4{va[4 * j], va[4 * j + 1], va[4 * j + 2], va[4 * j + 3]};
-            *(int4*)&sB[buf][r * GB_RS + lk] =
-                int4{vb[4 * j], vb[4 * j + 1], vb[4 * j + 2], vb[4 * j + 3]};
-        }
-    };
-    // S > 0: this lane's direct loads: rows 32 wave + lane / 4 (+ 16) of
+    // this lane's direct loads: rows 32 wave + lane / 4 (+ 16) of
     // A and B, the global chunk stored at position lane % 4 of its row
     int8_t* const stg = (int8_t*)gb_dyn;
     const int lrow = 32 * wave + (lane >> 2);
@@ -159,24 +107,14 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
 #pragma unroll
     for (int j = 0; j < 3; ++j)
         tv[j] = ((const int*)((const char*)a.plan + PLAN_E))[tid + 256 * j];
-    if constexpr (S > 0) {
-        // the first S - 1 steps in flight: they overlap the set-up below
+    // the first S - 1 steps in flight: they overlap the set-up below
 #pragma unroll
-        for (int sl = 0; sl < S - 1; ++sl)
-            if (sl < nk) dload(sl);
-    } else {
-        // every slot's loads first: they overlap the table set-up below
-#pragma unroll
-        for (int sl = 0; sl < P; ++sl) gload(ra[sl], rb[sl], sl);
-    }
+    for (int sl = 0; sl < S - 1; ++sl)
+        if (sl < nk) dload(sl);
 
-    // tables of the plan (S > 0: stored after the K loop, since an LDS
-    // store here would wait for the direct loads in flight) and the lane's
-    // 4 channels' constants
-    if constexpr (S == 0) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) s_tab[tid + 256 * j] = tv[j];
-    }
+    // tables of the plan (stored after the K loop, since an LDS store here
+    // would wait for the direct loads in flight) and the lane's 4 channels'
+    // constants
     const int4 hdr = *(const int4*)a.plan;
     // the lane's 4 channels' constants, the zero-point correction folded
     // into the plan constant (plan_q0; K <= 16384 keeps |w| + |corr| +
@@ -202,32 +140,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     int psum[4] = {0, 0, 0, 0};  // stored-byte sums of the lane's A rows
-    // one K-step (BK / 64 MFMA depths) from LDS buffer buf
-    auto mfma_step = [&](int buf, int ks) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < BK / 64; ++h) {
-            v4i fa[4], fb[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                fa[i] = *(const v4i*)&sA[buf][(64 * wm + 16 * i + col) *
-                                                  GB_RS + 64 * h + 16 * kg];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                fb[j] = *(const v4i*)&sB[buf][(64 * wn + 16 * j + col) *
-                                                  GB_RS + 64 * h + 16 * kg];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                        fa[i], fb[j], acc[i][j], 0, 0, 0);
-            if (RS && ks * GB_K + 64 * h + 16 * kg < kx) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) psum[i] += bytes_sum(fa[i], 16);
-            }
-        }
-    };
-    // S > 0: a lane's fragment of rows 16 i + col, chunk kg, at position
+    // a lane's fragment of rows 16 i + col, chunk kg, at position
     // kg ^ ((col >> 1) & 3) of the row (the tile's row bases are multiples
     // of 16)
     const int foff = col * 64 + 16 * (kg ^ ((col >> 1) & 3));
@@ -251,42 +164,25 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
             for (int i = 0; i < 4; ++i) psum[i] += bytes_sum(fa[i], 16);
         }
     };
-    if constexpr (S > 0) {
-        // step ks: this wave's loads of it done (those of the next
-        // min(S - 2, nk - 1 - ks) steps may still be in flight), barrier
-        // (every wave's part landed, and every wave is past step ks - 1,
-        // whose stage the refill below overwrites), request step
-        // ks + S - 1, MFMAs
-        for (int ks = 0; ks < nk; ++ks) {
-            wait_vm(4 * min(S - 2, nk - 1 - ks));
-            // a bare barrier: the explicit wait above is the only one the
-            // direct loads need (a fenced barrier would wait for all of
-            // them); the empty asm keeps LDS accesses on their side of it
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if (ks + S - 1 < nk) dload(ks + S - 1);
-            mfma_stage(stg + (ks % S) * GB_STAGE, ks);
-        }
-#pragma unroll
-        for (int j = 0; j < 3; ++j) s_tab[tid + 256 * j] = tv[j];
-        __syncthreads();
-    } else
-    // step ks from slot sl: to LDS buffer ks & 1 (last read two steps ago,
-    // before the previous step's barrier), refill the slot with step
-    // ks + P, barrier, MFMAs
-    for (int k0 = 0; k0 < nk; k0 += P) {
-#pragma unroll
-        for (int sl = 0; sl < P; ++sl) {
-            const int ks = k0 + sl;
-            if (ks < nk) {
-                sstore(ra[sl], rb[sl], ks & 1);
-                if (ks + P < nk) gload(ra[sl], rb[sl], ks + P);
-                __syncthreads();
-                mfma_step(ks & 1, ks);
-            }
-        }
+    // step ks: this wave's loads of it done (those of the next
+    // min(S - 2, nk - 1 - ks) steps may still be in flight), barrier
+    // (every wave's part landed, and every wave is past step ks - 1,
+    // whose stage the refill below overwrites), request step
+    // ks + S - 1, MFMAs
+    for (int ks = 0; ks < nk; ++ks) {
+        wait_vm(4 * min(S - 2, nk - 1 - ks));
+        // a bare barrier: the explicit wait above is the only one the
+        // direct loads need (a fenced barrier would wait for all of
+        // them); the empty asm keeps LDS accesses on their side of it
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (ks + S - 1 < nk) dload(ks + S - 1);
+        mfma_stage(stg + (ks % S) * GB_STAGE, ks);
     }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s_tab[tid + 256 * j] = tv[j];
+    __syncthreads();
 
     // epilogue: lane holds rows 16 i + 4 kg + r, column 16 j + col; the
     // quad's 4 channels of one row go out as one word (lane q of a quad
@@ -412,39 +308,26 @@ bool launch_gemm_big(const ConvArgs& b, hipStream_t st, int stages) {
         set_error("launch_gemm_big", "grid too large");
         return false;
     }
-    const int K = b.KGp * 16;
     const dim3 grid((unsigned)tiles);
     const int flags = (b.res ? 1 : 0) | (b.y2 ? 2 : 0) | (b.rowsum ? 4 : 0);
-    auto go = [&](auto kp, auto kbk, auto ks) {
-        constexpr int KP = decltype(kp)::value, KBK = decltype(kbk)::value;
+    auto go = [&](auto ks) {
         constexpr int KS = decltype(ks)::value;
         const size_t lds = (size_t)KS * GB_STAGE;
         switch (flags) {
-#define QA_GB_CASE(F)                                                    \
-    case F:                                                              \
-        k_gemm_big<KP, KBK, (F & 1) != 0, (F & 2) != 0, (F & 4) != 0, KS> \
-            <<<grid, 256, lds, st>>>(b);                                 \
+#define QA_GB_CASE(F)                                             \
+    case F:                                                       \
+        k_gemm_big<(F & 1) != 0, (F & 2) != 0, (F & 4) != 0, KS>  \
+            <<<grid, 256, lds, st>>>(b);                          \
         break;
             QA_GB_CASE(0) QA_GB_CASE(1) QA_GB_CASE(2) QA_GB_CASE(3)
             QA_GB_CASE(4) QA_GB_CASE(5) QA_GB_CASE(6) QA_GB_CASE(7)
 #undef QA_GB_CASE
         }
     };
-    // 128-byte steps when K allows, else 64-byte steps, the next step's
-    // loads in flight (measured on the ViT-S GEMMs: deeper rings, which
-    // cost VGPRs and so occupancy, were not faster in the pass)
-    // or (stages 3 / 4) the direct-to-LDS pipeline of 64-byte steps
-    using I1 = std::integral_constant<int, 1>;
-    using I0 = std::integral_constant<int, 0>;
-    using B64 = std::integral_constant<int, 64>;
-    if (stages == 3)
-        go(I1{}, B64{}, std::integral_constant<int, 3>{});
-    else if (stages == 4)
-        go(I1{}, B64{}, std::integral_constant<int, 4>{});
-    else if (K % 128 == 0)
-        go(I1{}, std::integral_constant<int, 128>{}, I0{});
+    if (stages == 4)
+        go(std::integral_constant<int, 4>{});
     else
-        go(I1{}, B64{}, I0{});
+        go(std::integral_constant<int, 3>{});
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_hip_error("launch_gemm_big", e);

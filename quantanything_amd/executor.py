@@ -2296,9 +2296,8 @@ class DeviceExecutor:
         out = [0]
         if d.H == d.W == d.KH == d.KW == 1 and d.G == 1 and \
                 d.w_layout == 0 and d.C % 16 == 0:
-            # the large-GEMM kernel (128 x 128 blocks): K steps staged
-            # through registers, or through 3 / 4 LDS stages of direct loads
-            out += [0x10400, 0x10403, 0x10404]
+            # the large-GEMM kernel: its own choice of blocks, then each
+            out += [0x10400, 0x10403, 0x10404, 0x10410, 0x10411, 0x10412]
         if DeviceExecutor.narrow_ok(d):
             # narrow GEMM: a 16 x 16 block a wave, 1, 2 or 4 row tiles a
             # wave with the same weights

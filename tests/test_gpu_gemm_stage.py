@@ -1,0 +1,35 @@
+"""The staged large-GEMM blocks (64 x 128, 128 x 128, 256 x 128, 256 x 256)
+against 64-bit integers: one row or column past and short of a block, and K of
+one step up to more steps than the deepest ring has stages."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1, 16, 1), (63, 64, 127), (65, 128, 129), (127, 192, 96),
+    (128, 256, 128), (129, 320, 131), (255, 336, 257), (256, 384, 256),
+    (257, 448, 255), (512, 576, 512), (300, 1040, 70), (1025, 640, 260)])
+def test_staged_blocks_bit_exact(hip, m, k, n):
+    import torch
+
+    from quantanything_amd.workloads import GemmWorkload
+
+    w = GemmWorkload(seed=m + n, M=m, K=k, N=n)
+    w.y = torch.full((m * n + 64,), 77, dtype=torch.int8, device="cuda")
+    w.d.y = w.y.data_ptr()
+    g = w.spec
+    acc = (g["a"].astype(np.int64) - g["zp_in"]) @ g["w"].astype(np.int64)
+    t = 31 + g["shift"]
+    q = ((acc + g["bias"]) * g["mult"] + (1 << (t - 1))) >> t
+    want = (np.clip(q + g["zp_out"], g["qmin"], g["qmax"]) - 128)
+    for code in (0, 0x10400, 0x10403, 0x10404, 0x10410, 0x10411, 0x10412):
+        w.d.tile = code
+        w.y.fill_(77)
+        w.launch()
+        got = w.y.cpu().numpy()
+        np.testing.assert_array_equal(got[:m * n].reshape(m, n), want,
+                                      err_msg=hex(code))
+        assert (got[m * n:] == 77).all(), hex(code)
