@@ -141,6 +141,18 @@ __host__ __device__ __forceinline__ float qa_f32_tie(int64_t zp, int64_t qmin,
     return (float)(0.5 - (double)(2 * w + 2) * 0x1p-22);
 }
 
+// The rounded quotient of qa_quantize_f32x2 below, in float32: the rounding
+// of x / scale where *slow stays as it is.
+__host__ __device__ __forceinline__ float qa_round_f32x2(float x, float invf,
+                                                         float invlo,
+                                                         bool* slow) {
+    const float r = rintf(x * invf);
+    const float d = fmaf(x, invlo, fmaf(x, invf, -r));
+    const float ad = fabsf(d);
+    *slow |= !(fabsf(ad - 0.5f) > 0x1p-22f) || !(ad < 1.0f);
+    return r + rintf(d);
+}
+
 // qa_quantize_f32 with the reciprocal in two floats, invf = float(inv) and
 // invlo = float(inv - invf), for callers whose waves quantize many values
 // at once: there the one-float form's tie zone (2^-12 of all values of an
@@ -150,18 +162,18 @@ __host__ __device__ __forceinline__ float qa_f32_tie(int64_t zp, int64_t qmin,
 // r = rint(x * invf), so that x * invf - r is below 0.57 and rounded by
 // 2^-25; adding x * invlo (below 2^-4) rounds by 2^-25 again, and
 // x (invf + invlo) is x / scale to 2^-48 relatively: d is the distance of
-// x / scale from r to within 2^-23. So r + rint(d) is the rounded quotient
-// unless |d| lies within 2^-22 of 1/2 (or is NaN, x infinite among the
-// cases): *slow. Beyond 2^20 the sum with zp is past the clip bounds, which
-// lie within 2^19 of zp, either way.
+// x / scale from r to within 2^-23, and below 1. So r + rint(d) is the
+// rounded quotient unless |d| lies within 2^-22 of 1/2: *slow, which an |d|
+// of 1 or more sets as well: infinities and NaN, and every finite x whose
+// x * invf overflows float32 (r infinite, d too, their sum NaN). Beyond 2^20
+// and not *slow, the sum with zp is past the clip bounds, which lie within
+// 2^19 of zp, either way.
 __device__ __forceinline__ int qa_quantize_f32x2(float x, float invf,
                                                  float invlo, int zp,
                                                  int qmin, int qmax,
                                                  bool* slow) {
-    const float r = rintf(x * invf);
-    const float d = fmaf(x, invlo, fmaf(x, invf, -r));
-    *slow |= !(fabsf(fabsf(d) - 0.5f) > 0x1p-22f);
-    return (int)__builtin_amdgcn_fmed3f(r + rintf(d) + (float)zp, (float)qmin,
+    const float q = qa_round_f32x2(x, invf, invlo, slow);
+    return (int)__builtin_amdgcn_fmed3f(q + (float)zp, (float)qmin,
                                         (float)qmax);
 }
 

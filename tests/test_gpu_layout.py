@@ -59,3 +59,33 @@ def test_planes_round_trip(hip, code, n, c, hw, sp, shift):
         np.testing.assert_array_equal(out[:n * (c - c0) * hw],
                                       back.reshape(-1))
         assert (out[n * (c - c0) * hw:] == 5.0).all()
+
+
+@pytest.mark.parametrize("code,c,hw,sp", [
+    (1, 40, 36, 48), (1, 7, 9, 7),     # tiles; any pixel stride
+    (2, 40, 36, 40), (2, 3, 20, 4)])   # tiles; four pixels a thread
+@pytest.mark.parametrize("scale", [2.0**-60, 1e-12, 0.037, 2.0**60])
+def test_values_past_float32_quotients(hip, code, c, hw, sp, scale):
+    """Finite values whose quotient by the scale passes float32 saturate on
+    their own side."""
+    import torch
+
+    dt, so, qmin, qmax = CODES[code]
+    zp = 130
+    top = np.finfo(np.float32).max
+    ext = np.array([top, 3.4e38, 1e38, 1.3e37, 1e37, 1e30, 1e20, 0.0,
+                    np.inf], np.float32)
+    x = np.resize(np.concatenate([ext, -ext, [np.nan]]),
+                  (2, c, hw)).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    y = torch.full((2 * hw * sp,), 77, dtype=torch.int8 if code == 1
+                   else torch.int16, device="cuda")
+    assert hip.library().qa_d_quantize_nhwc(
+        xd.data_ptr(), 2, c, hw, y.data_ptr(), code, sp, scale, zp, qmin,
+        qmax, so, torch.cuda.current_stream().cuda_stream) == 0
+    with np.errstate(invalid="ignore"):
+        v = np.rint(x.astype(np.float64) / scale) + zp
+        q = np.where(np.isnan(v), -2.0**31, np.clip(v, qmin, qmax))
+    want = (q.astype(np.int64) - so).astype(dt)
+    got = y.cpu().numpy().reshape(2, hw, sp)
+    np.testing.assert_array_equal(got[:, :, :c], want.transpose(0, 2, 1))
