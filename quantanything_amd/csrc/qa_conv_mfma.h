@@ -267,6 +267,20 @@ __device__ __forceinline__ int64_t quant_general(const ConvArgs& a,
     return q;
 }
 
+// A work-group barrier that waits for this wave's LDS accesses but its N
+// newest (reads and writes complete in issue order; N 0..15), and for
+// nothing else: the barrier alone waits for no memory, and a fenced one
+// (__syncthreads) would wait for direct loads still in flight. The empty asm
+// keeps LDS accesses on their side of it.
+template <int N = 0>
+__device__ __forceinline__ void lds_barrier() {
+    static_assert(N >= 0 && N <= 15, "lgkmcnt has 4 bits");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f | N << 8);  // lgkmcnt(N)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // med3(x, lo, hi) = clip(x, lo, hi) for lo <= hi, as one VALU instruction
 // (the compiler otherwise emits a max and a min).
 __device__ __forceinline__ int med3_i32(int x, int lo, int hi) {

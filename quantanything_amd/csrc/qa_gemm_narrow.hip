@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
         cbo[r] = RS ? (uint32_t)a.boff[c] : 0u;
     }
     // every load done (the direct ones among them), the table to LDS, then
-    // one bare barrier (the empty asm keeps LDS accesses on their side)
+    // one barrier that waits for these LDS writes
     __builtin_amdgcn_s_waitcnt(0x0f70);
     s_tab[tid] = tv;
     if (CV && fix) {  // padding taps: the pad value over what was loaded
@@ -175,9 +175,7 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
             if ((fix >> k) & 1)
                 *(v4i*)(s_x + 1024 * i + 16 * lane) = v4i{pv, pv, pv, pv};
     }
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    lds_barrier();
     if (!WF) {
         const int8_t* fw0 =
             s_w + (c0 - cw + col) * 64 + 16 * (kg ^ ((col >> 2) & 3));

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(NC_NT) void k_narrow_chain(NcArgs a) {
 
     // the tables, constants and rows landed (loads complete in issue
     // order: conv 1's weights and conv 2's follow them); the padding taps'
-    // pad value; one bare barrier
+    // pad value, which the barrier waits for
     constexpr int NW = CT1 * KM1 + NW2;  // loads after the rows (<= 44)
     __builtin_amdgcn_s_waitcnt(0x0f70 | (NW & 15) | ((NW >> 4) << 14));
     if (CV1 && fix) {
@@ -200,9 +200,7 @@ __global__ __launch_bounds__(NC_NT) void k_narrow_chain(NcArgs a) {
             if ((fix >> k) & 1)
                 *(v4i*)(s_x + 1024 * i + 16 * lane) = v4i{pv, pv, pv, pv};
     }
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    lds_barrier();
 
     // the table epilogue of one accumulator: channels c + r of conv h
     auto epi = [&](int h, const v4i& acc, int c, const int4& hdr,
