@@ -167,6 +167,7 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
         k.add = (double)(a.ws_k[co] + (in ? pre : 0));
         s_ch[tid] = k;
     }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the direct loads landed
     __syncthreads();
 
     const int64_t ntiles = (a.M + 15) >> 4;

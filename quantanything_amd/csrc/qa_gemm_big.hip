@@ -171,12 +171,9 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
     // ks + S - 1, MFMAs
     for (int ks = 0; ks < nk; ++ks) {
         wait_vm(4 * min(S - 2, nk - 1 - ks));
-        // a bare barrier: the explicit wait above is the only one the
-        // direct loads need (a fenced barrier would wait for all of
-        // them); the empty asm keeps LDS accesses on their side of it
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        // (the direct loads are waited for above; a fenced barrier would
+        // wait for all of them)
+        lds_barrier();
         if (ks + S - 1 < nk) dload(ks + S - 1);
         mfma_stage(stg + (ks % S) * GB_STAGE, ks);
     }

@@ -171,14 +171,10 @@ __global__ __launch_bounds__(
         for (int i = 0; i < MT; ++i)
             f.a[i] = *(const v4i*)(sb + (16 * MT * wm + 16 * i) * 64);
     };
-    // a bare barrier: the explicit waits are the only ones the direct loads
-    // need (a fenced barrier would wait for all of them); the empty asm keeps
-    // LDS accesses on their side of it
-    auto barrier = [&]() __attribute__((always_inline)) {
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
+    // the waits are explicit: on the direct loads (wait_vm), and on this
+    // wave's fragment reads but those of the last step (lds_barrier)
+    constexpr int NF = MT + NT;  // fragment reads of a step
+    auto barrier = [&]() __attribute__((always_inline)) { lds_barrier<NF>(); };
     auto product = [&](const Frag& f, int ks) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -199,7 +195,8 @@ __global__ __launch_bounds__(
     // step ks from cur's registers, the next step's fragments read meanwhile:
     // this wave's loads of step ks + 1 done (those of the next S - 3 steps may
     // still be in flight), barrier (every wave's part landed, and every wave
-    // has the fragments of step ks - 1, whose stage the refill overwrites).
+    // has the fragments of step ks - 1, whose stage the refill overwrites:
+    // only the NF reads of step ks may still be in flight).
     // No branch between the reads and the MFMAs: at one the compiler waits
     // for every read.
     auto steady = [&](const Frag& cur, Frag& nxt, int ks)

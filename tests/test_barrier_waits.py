@@ -47,3 +47,26 @@ def test_lds_writes_are_waited_for(tmp_path, src):
                 assert not back.startswith("ds_write"), \
                     f"{name}: {back} still in flight at a barrier"
     assert barriers > 0
+
+
+def test_ring_reads_are_waited_for(tmp_path):
+    """A barrier of the staged GEMM's ring leaves no fragment read in flight
+    but those of the last step (MT + NT of them): the stage of the step
+    before is refilled right after it."""
+    barriers = 0
+    for name, ins in _kernels("qa_gemm_stage.hip", tmp_path).items():
+        bm, bn, wm, wn = map(int, re.search(
+            r"k_gemm_stageILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E", name).groups())
+        reads = bm // wm // 16 + bn // wn // 16
+        for at, text in enumerate(ins):
+            if not text.startswith("s_barrier"):
+                continue
+            barriers += 1
+            for back in reversed(ins[:at]):
+                wait = re.match(r"s_waitcnt.*lgkmcnt\((\d+)\)", back)
+                if wait:
+                    assert int(wait.group(1)) <= reads, name
+                    break
+                assert not back.startswith("ds_"), \
+                    f"{name}: {back} not waited for at a barrier"
+    assert barriers > 0
