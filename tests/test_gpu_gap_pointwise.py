@@ -46,6 +46,34 @@ def test_gap_rows(hip, code, n, c, hw, fill):
     assert (got[:, c:] == 9).all()
 
 
+@pytest.mark.parametrize("n,c,hw,sp,off", [
+    (3, 20, 49, 20, 0), (2, 64, 700, 68, 4), (1, 300, 3, 320, 12),
+    (2, 12, 3136, 24, 12), (2, 4, 1, 4, 0),  # words of 4 channels
+    (2, 18, 49, 20, 0), (2, 20, 49, 21, 1)])  # a channel a thread
+def test_gap_off_16_bytes(hip, n, c, hw, sp, off):
+    """Rows on 4 bytes alone (a Split half, a caller's dense rows) and on
+    none."""
+    import torch
+
+    rng = np.random.default_rng(c + hw)
+    x = rng.integers(-128, 128, (n, hw, sp)).astype(np.int8)
+    x = np.concatenate([x.reshape(-1), np.zeros(64, np.int8)])
+    zi, so, m, s, zo = 3, 1, 1400000000, 6, -2
+    xd = torch.from_numpy(x).cuda()
+    y = torch.full((n, c + 3), 9, dtype=torch.int8, device="cuda")
+    assert hip.library().qa_d_gap(
+        xd.data_ptr() + off, 1, hw * sp, 1, sp, n, c, hw, zi, so, m, s, zo,
+        -128, 127, y.data_ptr(), 1, c + 3, 0, None) == 0
+    rows = np.stack([x[off + i * hw * sp:][:hw * sp].reshape(hw, sp)[:, :c]
+                     for i in range(n)])
+    acc = rows.astype(np.int64).sum(1) + hw * (so - zi)
+    want = np.clip(multiply_by_quantized_multiplier(acc, m, s) + zo, -128,
+                   127)
+    got = y.cpu().numpy()
+    np.testing.assert_array_equal(got[:, :c], want.astype(np.int8))
+    assert (got[:, c:] == 9).all()
+
+
 @pytest.mark.parametrize("qt", ["int8", "uint8"])
 @pytest.mark.parametrize("cin,cout,size,form", [
     (64, 128, 19, "plain"), (128, 132, 16, "add"), (64, 200, 18, "concat"),
