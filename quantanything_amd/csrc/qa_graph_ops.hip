@@ -131,8 +131,9 @@ __global__ __launch_bounds__(TH) void k_gap_cl16(
     store_s(out, out_code, n * out_sn + g0 + tid, q - out_so);
 }
 
-// Channels-last int8 input on 4-byte strides that are not on 16 (a channel
-// half, a caller's own rows), C a multiple of 4: a thread sums 4 channels
+// Channels-last int8 input on 4-byte strides, C a multiple of 4 (few pixels,
+// many images, or rows that are not on 16 bytes: a channel half, a caller's
+// own rows): a thread sums 4 channels
 // (one word per pixel) over a quarter of the pixels (the 4 waves of a
 // work-group take pixels w, w+4, ...); the partial sums meet in LDS and wave
 // 0 requantizes and stores. 32x128x28x28 in rows of 256: 11.9 us, against
@@ -631,9 +632,28 @@ QA_API int qa_d_gap(const void* x, int in_code, int64_t x_sn, int64_t x_sc,
     hipStream_t st = (hipStream_t)stream;
     // 16-byte rows; sums in int32: |stored| HW < 2^31
     const int64_t ch = in_code == 2 ? 8 : 16;
-    if (x_sc == 1 && (in_code == 1 || in_code == 2) && x_sp % ch == 0 &&
-        x_sn % ch == 0 && (uintptr_t)x % 16 == 0 && C < (1 << 30) &&
-        HW < (in_code == 1 ? 1 << 23 : 1 << 15)) {
+    const bool words = x_sc == 1 && in_code == 1 && C % 4 == 0 &&
+                       x_sp % 4 == 0 && x_sn % 4 == 0 &&
+                       (uintptr_t)x % 4 == 0 && HW < (1 << 23);
+    bool rows16 = x_sc == 1 && (in_code == 1 || in_code == 2) &&
+                  x_sp % ch == 0 && x_sn % ch == 0 && (uintptr_t)x % 16 == 0 &&
+                  C < (1 << 30) && HW < (in_code == 1 ? 1 << 23 : 1 << 15);
+    // The 16-byte form spreads an image's pixels over a work-group's lanes
+    // and pays for their reduction: not for few pixels (int8 against words,
+    // us: 64x1280 of 7x7 7.4 / 4.0, of 10x10 7.5 / 4.7, 16x256 of 14x14 5.1 /
+    // 5.4, of 28x28 6.3 / 12.3; int16 against a thread a channel: 64x256 of
+    // 2x2 3.7 / 2.8, of 4x4 3.7 / 4.5, but 256x256 of 4x4 5.8 / 4.6), nor
+    // where words of 4 channels fill the 256 CUs, most lanes busy (256x256 of
+    // 28x28 23.4 / 19.8, 64x1280 27.2 / 22.5; 2048x64 31.2 / 38.6).
+    if (words) {
+        const int64_t wg = qa::ceil_div(C, 256);
+        rows16 = rows16 && HW > 128 &&
+                 !(C >= 192 * wg && N * wg >= 256);
+    } else {
+        rows16 = rows16 && HW > 8 &&
+                 !(HW <= 16 && N * qa::ceil_div(C, 4 * ch) >= 2048);
+    }
+    if (rows16) {
         if (N > 65535) {
             qa::set_error("qa_d_gap", "N above 65535");
             return -1;
@@ -654,8 +674,7 @@ QA_API int qa_d_gap(const void* x, int in_code, int64_t x_sn, int64_t x_sc,
             big ? go(int8_t{}, Big{}) : go(int8_t{}, Small{});
         else
             big ? go(int16_t{}, Big{}) : go(int16_t{}, Small{});
-    } else if (x_sc == 1 && in_code == 1 && C % 4 == 0 && x_sp % 4 == 0 &&
-               x_sn % 4 == 0 && (uintptr_t)x % 4 == 0 && HW < (1 << 23)) {
+    } else if (words) {
         if (N > 65535) {
             qa::set_error("qa_d_gap", "N above 65535");
             return -1;

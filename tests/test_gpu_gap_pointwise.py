@@ -48,11 +48,13 @@ def test_gap_rows(hip, code, n, c, hw, fill):
 
 @pytest.mark.parametrize("n,c,hw,sp,off", [
     (3, 20, 49, 20, 0), (2, 64, 700, 68, 4), (1, 300, 3, 320, 12),
-    (2, 12, 3136, 24, 12), (2, 4, 1, 4, 0),  # words of 4 channels
-    (2, 18, 49, 20, 0), (2, 20, 49, 21, 1)])  # a channel a thread
-def test_gap_off_16_bytes(hip, n, c, hw, sp, off):
+    (2, 12, 3136, 24, 12), (2, 4, 1, 4, 0), (300, 256, 130, 256, 0),
+    (3, 128, 128, 128, 0), (3, 128, 129, 128, 0),  # words of 4 channels
+    (2, 18, 49, 20, 0), (2, 20, 49, 21, 1), (2, 18, 8, 32, 0),
+    (700, 130, 16, 144, 0)])  # a channel a thread
+def test_gap_words_and_channels(hip, n, c, hw, sp, off):
     """Rows on 4 bytes alone (a Split half, a caller's dense rows) and on
-    none."""
+    none, few pixels and many images."""
     import torch
 
     rng = np.random.default_rng(c + hw)
