@@ -376,8 +376,14 @@ template <class T>
 void launch_maxpool_cl(const qa_maxpool_desc& d, hipStream_t st) {
     const int64_t nch = ceil_div(d.C, 16 / (int64_t)sizeof(T));
     const int64_t outs = d.N * d.OH * d.OW;
-    // many taps and few outputs: a work-group an output
-    if (d.KH * d.KW >= 64 && outs * nch < 65536) {
+    // Many taps and few outputs: a work-group an output (taps without an
+    // unrolled form in a thread, one after the other, against it, us: 64x512
+    // of 7x7 -> 1x1 12.1 / 3.9, 4x4 windows of 32x256x32x32, 32768 chunks
+    // of outputs, 5.6 / 5.0, 7x7 of 16x128x20x20, 51200, 11.4 / 13.4).
+    const int64_t taps = d.KH * d.KW;
+    const bool unrolled = d.KH == 5 && d.KW == 5;
+    if ((taps >= 64 && outs * nch < 65536) ||
+        (taps >= 16 && !unrolled && outs * nch <= 32768)) {
         int cb = 1;
         while (cb < nch && cb < 16) cb *= 2;
         const dim3 g((unsigned)outs, (unsigned)ceil_div(nch, cb));

@@ -30,7 +30,12 @@ def _dev(a):
     (1, 24, 9, 11, (3, 5), (1, 1), (1, 1), (1, 2)),
     (3, 40, 23, 21, (23, 21), (1, 1), (1, 1), (0, 0)),  # the whole image
     (2, 16, 20, 20, (9, 9), (3, 3), (1, 1), (4, 4)),
-    (1, 300, 9, 8, (9, 8), (1, 1), (1, 1), (0, 0))])
+    (1, 300, 9, 8, (9, 8), (1, 1), (1, 1), (0, 0)),
+    (5, 72, 7, 7, (7, 7), (1, 1), (1, 1), (0, 0)),  # a work-group an output
+    (2, 24, 11, 12, (4, 4), (2, 2), (1, 1), (1, 1)),
+    (3, 33, 8, 9, (2, 8), (1, 1), (2, 1), (0, 2)),
+    (9, 256, 17, 16, (4, 5), (1, 1), (1, 1), (2, 2)),  # 41472, 82944 chunks
+    (2, 16, 9, 9, (5, 3), (2, 2), (1, 1), (1, 1))])
 @pytest.mark.parametrize("high", [False, True])
 def test_maxpool_chunks(hip, code, n, c, h, w, k, s, dl, pad, high):
     t = TYPES[code]
