@@ -207,6 +207,22 @@ __device__ __forceinline__ int64_t qa_quantize_mixed(float x, bool f32ok,
     return qa_quantize_one_fast(x, scale, inv, zp, qmin, qmax);
 }
 
+namespace qa {
+
+// Whether 16 bytes of a row a thread (the row kernels of the copies and
+// Pads) beat an element a thread, for int8 or int16 and that many elements
+// in all: below, one element each in as many threads as the chip holds is
+// the shorter chain, in three or four axes less so for their index
+// arithmetic. us, element / row kernel: int8 2000x500 padded to 2000x502 4.8 / 4.3,
+// 500x500 2.9 / 4.2, rows of 17 copied 64000 of them 6.5 / 4.6, 16000 3.5 / 4.0,
+// 8x24x60x60 channel halves 7.1 / 4.7, 2x24x60x60 3.9 / 4.3; int16 2000x500
+// 4.9 / 4.0, 500x500 2.9 / 3.5, 2x24x60x60 4.5 / 3.2, 8x20x14x14 3.4 / 3.7.
+inline bool rows16_pay(int64_t code, int64_t ndim, int64_t total) {
+    return total * code >= (ndim > 2 ? (int64_t)1 << 18 : (int64_t)3 << 18);
+}
+
+}  // namespace qa
+
 // --------------------------------------------------------------- errors ---
 namespace qa {
 

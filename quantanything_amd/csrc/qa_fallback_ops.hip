@@ -618,7 +618,8 @@ QA_API int qa_d_copy_nd(const qa_nd_copy* d, void* stream) {
         return launched("qa_d_copy_nd") ? 0 : -1;
     }
     qa_nd_pad p;
-    if (copy_as_pad(*d, &p)) return qa_d_pad_nd(&p, stream);
+    if (rows16_pay(d->x_code, d->ndim, total) && copy_as_pad(*d, &p))
+        return qa_d_pad_nd(&p, stream);
     const int64_t blocks = std::min<int64_t>(ceil_div(total, kThreads), 65535);
     if (total < ((int64_t)1 << 32))  // every extent divides in 32 bits
         k_copy_nd<true><<<(unsigned)blocks, kThreads, 0,

@@ -464,7 +464,7 @@ QA_API int qa_d_pad_nd(const qa_nd_pad* d, void* stream) {
         small = small && o.shape[k] < (1 << 30) && o.lo[k] < (1 << 30) &&
                 o.xshape[k] < (1 << 30);
     if (o.ys[last] == 1 && o.xs[last] == 1 && small && o.code <= 2 &&
-        o.shape[last] >= ch) {
+        o.shape[last] >= ch && rows16_pay(o.code, o.ndim, total)) {
         const unsigned g = (unsigned)std::min<int64_t>(
             ceil_div(rows * chunks, kThreads), 1 << 20);
         if (o.code == 1)

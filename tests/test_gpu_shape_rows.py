@@ -8,7 +8,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from quantanything_amd.executor import MaxPoolDesc, PadDesc
+from quantanything_amd.executor import MaxPoolDesc, NdCopy, PadDesc
 from quantanything_amd.utils import multiply_by_quantized_multiplier
 
 pytestmark = pytest.mark.gpu
@@ -74,7 +74,11 @@ def test_maxpool_chunks(hip, code, n, c, h, w, k, s, dl, pad, high):
     ((3, 20, 4, 5), (1, 0, 0, 3), (0, 5, 2, 0), (0, 2, 3, 1)),
     ((2, 5, 6, 40), (0, 1, 1, 7), (1, 0, 1, 9), (0, 1, 2, 3)),
     ((4, 33), (2, 3), (1, 2), (0, 1)), ((33, 18), (0, 4), (1, 1), (1, 0)),
-    ((2, 3, 4, 17), (0, 0, 0, 16), (0, 0, 0, 1), (3, 1, 0, 2))])
+    ((2, 3, 4, 17), (0, 0, 0, 16), (0, 0, 0, 1), (3, 1, 0, 2)),
+    # past the size from which a thread takes 16 bytes of a row
+    ((4, 70, 33, 31), (0, 2, 1, 2), (0, 1, 2, 1), (0, 2, 3, 1)),
+    ((1500, 533), (2, 3), (1, 2), (0, 1)),
+    ((533, 1500), (0, 4), (1, 1), (1, 0))])
 def test_pad_rows(hip, code, shape, lo, hi, order):
     t = TYPES[code]
     rng = np.random.default_rng(sum(shape))
@@ -98,6 +102,41 @@ def test_pad_rows(hip, code, shape, lo, hi, order):
     np.testing.assert_array_equal(
         got[:ym.size].reshape(ym.shape), want.transpose(order))
     assert (got[ym.size:] == 9).all()
+
+
+@pytest.mark.parametrize("code", [1, 2])
+@pytest.mark.parametrize("shape,xst,yst,off", [
+    ((3, 17, 4, 5), (640, 1, 160, 32), (480, 1, 120, 24), 5),
+    ((9, 31, 40, 41), (104960, 1, 2624, 64), (82000, 1, 2050, 50), 31),
+    ((2, 24, 90, 91), (0, 1, 4368, 48), (262080, 1, 2912, 32), 24),
+    ((1700, 501), (512, 1), (503, 1), 1), ((30, 37), (37, 1), (64, 1), 0),
+    ((501, 1700), (1, 512), (1, 503), 3), ((40, 9000), (9001, 1), (9000, 1), 0),
+    # the output's rows not contiguous, or its other axis at stride 1
+    ((900, 900), (900, 1), (1801, 2), 0), ((900, 1), (16, 1), (1, 1), 0)])
+def test_copy_rows(hip, code, shape, xst, yst, off):
+    """Plain copies of views off the 16-byte grid (a Split's half, a batch
+    read again from one image, odd matrices), on each side of the size from
+    which a thread takes 16 bytes of a row."""
+    import torch
+
+    t = TYPES[code]
+    info = np.iinfo(t)
+    rng = np.random.default_rng(sum(shape))
+    size = off + 1 + sum((n - 1) * s for n, s in zip(shape, xst))
+    x = rng.integers(info.min, info.max + 1, size).astype(t)
+    ysize = 1 + sum((n - 1) * s for n, s in zip(shape, yst))
+    xd, yd = _dev(x), _dev(np.full(ysize + 40, 55, t))
+    d = NdCopy()
+    d.x, d.x_code = xd.data_ptr() + off * code, code
+    d.y, d.y_code, d.ndim = yd.data_ptr(), code, len(shape)
+    for k, v in enumerate(zip(shape, xst, yst)):
+        d.shape[k], d.xs[k], d.ys[k] = v
+    d.qmin, d.qmax = -(1 << 62), 1 << 62
+    assert hip.library().qa_d_copy_nd(ctypes.byref(d), None) == 0
+    want = torch.full((ysize + 40,), 55, dtype=yd.dtype)
+    torch.as_strided(want, shape, yst).copy_(
+        torch.as_strided(torch.from_numpy(x), shape, xst, off))
+    np.testing.assert_array_equal(yd.cpu().numpy(), want.numpy())
 
 
 @pytest.mark.parametrize("rows,cols,xs,ys,m,s,qmin,qmax", [
