@@ -120,6 +120,7 @@ __global__ __launch_bounds__(kThreads) void k_quantize_any(
 #pragma unroll
         for (int k = 0; k < CH; ++k) {
             const float* s = x + (n * C + min(c0 + k, C - 1)) * HW + p;
+            if (c0 + k >= C) continue;
             if constexpr (PX == 4) {
                 const float4 v = *(const float4*)s;
                 f[k][0] = v.x;
@@ -135,10 +136,12 @@ __global__ __launch_bounds__(kThreads) void k_quantize_any(
         for (int j = 0; j < PX; ++j)
 #pragma unroll
             for (int k = 0; k < CH; ++k) {
+                q[j][k] = (T)0;
+                if (c0 + k >= C) continue;
                 bool slow = !o.f32ok;
                 int v = quant_f32(o, f[k][j], &slow);
                 if (__builtin_expect(slow, 0)) v = quant_f64(o, f[k][j]);
-                q[j][k] = c0 + k < C ? (T)v : (T)0;
+                q[j][k] = (T)v;
             }
         T* d = y + (n * HW + p) * y_sp + c0;
         if constexpr (PX == 4) {  // y_sp == CH: the pixels are contiguous
@@ -269,7 +272,10 @@ bool quantize_planes(const float* x, int64_t N, int64_t C, int64_t HW, T* y,
         if (row == 32) return go(std::integral_constant<int, 32>{});
         return go(std::integral_constant<int, 64>{});
     }
+    // (four pixels a thread once single ones fill the chip: 3 channels of
+    // 32x224x224 10.4 -> 7.3 us, but of 1x224x224 2.8 -> 3.3)
     const bool four = sizeof(T) == 2 && y_sp == 4 && HW % 4 == 0 &&
+                      pixels >= (1 << 18) &&
                       ((uintptr_t)x | (uintptr_t)y) % 16 == 0;
     const int64_t groups = four ? pixels / 4 : pixels;
     const int64_t nch = ceil_div(y_sp, 4);

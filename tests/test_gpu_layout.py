@@ -16,7 +16,9 @@ CODES = {1: (np.int8, 128, 0, 255), 2: (np.int16, 32768, 0, 65535)}
     (1, 1, 5, 1, 16, 0), (1, 2, 24, 57 * 57, 32, 0), (1, 3, 16, 12, 16, 0),
     (1, 8, 64, 56 * 56, 64, 0),  # four pixels a thread
     (1, 2, 7, 9, 7, 0), (1, 2, 20, 10, 21, 1),  # element stores
-    (2, 3, 3, 224 * 224, 4, 0), (2, 2, 9, 25, 9, 0), (2, 2, 24, 49, 24, 0),
+    (2, 3, 3, 224 * 224, 4, 0), (2, 2, 9, 25, 9, 0),
+    (2, 6, 3, 224 * 224, 4, 0), (2, 340, 1, 784, 4, 0),  # four pixels
+    (2, 5, 1, 784, 4, 0), (2, 2, 2, 9, 4, 0), (2, 2, 24, 49, 24, 0),
     (2, 1, 8, 64, 8, 1), (2, 64, 40, 36, 40, 0)])
 def test_planes_round_trip(hip, code, n, c, hw, sp, shift):
     import torch
@@ -63,7 +65,8 @@ def test_planes_round_trip(hip, code, n, c, hw, sp, shift):
 
 @pytest.mark.parametrize("code,c,hw,sp", [
     (1, 40, 36, 48), (1, 7, 9, 7),     # tiles; any pixel stride
-    (2, 40, 36, 40), (2, 3, 20, 4)])   # tiles; four pixels a thread
+    (2, 40, 36, 40), (2, 3, 20, 4),    # tiles; one pixel a thread
+    (2, 3, 1 << 17, 4)])               # four
 @pytest.mark.parametrize("scale", [2.0**-60, 1e-12, 0.037, 2.0**60])
 def test_values_past_float32_quotients(hip, code, c, hw, sp, scale):
     """Finite values whose quotient by the scale passes float32 saturate on
