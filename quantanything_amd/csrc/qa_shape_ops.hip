@@ -165,12 +165,22 @@ struct MaxAcc {
     }
 };
 
-// 16 bytes of channels at p; the chunk's last elements may not exist
+// The end of the tensor's last element. 16 bytes that end before it lie
+// between its first and last element, whatever they hold past a pixel's
+// channels (maxpool_cl_ok: no negative strides).
+template <class T>
+__device__ __forceinline__ const T* pool_end(const qa_maxpool_desc& d) {
+    return (const T*)d.x + (d.N - 1) * d.x_sn + (d.H - 1) * d.x_sh +
+           (d.W - 1) * d.x_sw + d.C;
+}
+
+// 16 bytes of channels at p, the first `real` of them the pixel's (the
+// others anything); element loads where the tensor ends within them
 template <class T>
 __device__ __forceinline__ void load_chunk(const T* p, int real,
-                                           uint32_t* w) {
+                                           const T* end, uint32_t* w) {
     constexpr int CH = 16 / sizeof(T);
-    if (real >= CH) {
+    if (real >= CH || p + CH <= end) {
         const uint4 v = *(const uint4*)p;
         w[0] = v.x;
         w[1] = v.y;
@@ -205,12 +215,14 @@ __device__ __forceinline__ void store_chunk(T* p, int real, uint4 v) {
 // K: a K x K window, its taps unrolled so that all loads are in flight
 // where a whole wave's windows lie inside the image; 0: any window.
 // 16x32x112x112, 5x5 (12.8 MB moved, 25 taps from L1): 12.6 us; 105 us with
-// a channel a thread.
+// a channel a thread. A last chunk of fewer channels is loaded whole
+// (8x100x20x20, 5x5: 6.1 us, 14.7 us by elements).
 template <class T, int K>
 __global__ __launch_bounds__(kThreads) void k_maxpool_cl(qa_maxpool_desc d,
                                                          uint32_t nch,
                                                          uint32_t total) {
     constexpr int CH = 16 / sizeof(T);
+    const T* const end = pool_end<T>(d);
     for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < total;
          i += gridDim.x * kThreads) {
         uint32_t r = i / nch;
@@ -226,9 +238,12 @@ __global__ __launch_bounds__(kThreads) void k_maxpool_cl(qa_maxpool_desc d,
         const int ix0 = ox * (int)d.SW - (int)d.PL;
         const T* xb = (const T*)d.x + n * d.x_sn + c;
         MaxAcc<T> acc;
-        const bool in = iy0 >= 0 && ix0 >= 0 && real >= CH &&
-                        iy0 + (KH - 1) * (int)d.DH < (int)d.H &&
-                        ix0 + (KW - 1) * (int)d.DW < (int)d.W;
+        const int iy1 = iy0 + (KH - 1) * (int)d.DH;
+        const int ix1 = ix0 + (KW - 1) * (int)d.DW;
+        const bool in = iy0 >= 0 && ix0 >= 0 && iy1 < (int)d.H &&
+                        ix1 < (int)d.W &&
+                        (real >= CH ||
+                         xb + iy1 * d.x_sh + ix1 * d.x_sw + CH <= end);
         if (K > 0 && __all(in)) {
             const T* p = xb + iy0 * d.x_sh + ix0 * d.x_sw;
             uint4 v[K > 0 ? K * K : 1];
@@ -257,7 +272,8 @@ __global__ __launch_bounds__(kThreads) void k_maxpool_cl(qa_maxpool_desc d,
                     const int ix = ix0 + kx * (int)d.DW;
                     uint32_t w[4];
                     if (row_in && (uint32_t)ix < (uint32_t)d.W) {
-                        load_chunk(xb + iy * d.x_sh + ix * d.x_sw, real, w);
+                        load_chunk(xb + iy * d.x_sh + ix * d.x_sw, real, end,
+                                   w);
                     } else {
                         const uint32_t u =
                             sizeof(T) == 1
@@ -305,6 +321,7 @@ __global__ __launch_bounds__(kThreads) void k_maxpool_wide(qa_maxpool_desc d,
     const int iy0 = oy * (int)d.SH - (int)d.PT;
     const int ix0 = ox * (int)d.SW - (int)d.PL;
     const T* xb = (const T*)d.x + n * d.x_sn + c;
+    const T* const end = pool_end<T>(d);
     const int taps = (int)(d.KH * d.KW);
     // a thread without taps repeats the first one
     auto tap = [&](int t, uint32_t* w) {
@@ -313,7 +330,7 @@ __global__ __launch_bounds__(kThreads) void k_maxpool_wide(qa_maxpool_desc d,
         const bool in = (uint32_t)iy < (uint32_t)d.H &&
                         (uint32_t)ix < (uint32_t)d.W;
         if (in) {
-            load_chunk(xb + iy * d.x_sh + ix * d.x_sw, real, w);
+            load_chunk(xb + iy * d.x_sh + ix * d.x_sw, real, end, w);
         } else {
             const uint32_t u = sizeof(T) == 1
                                    ? (uint32_t)(uint8_t)d.pad * 0x01010101u
@@ -354,13 +371,14 @@ __global__ __launch_bounds__(kThreads) void k_maxpool_wide(qa_maxpool_desc d,
 }
 
 // Whether the 16-byte channel kernels take a pool: channels contiguous, every
-// other stride and both bases on 16 bytes, extents and indices in 32 bits.
+// other stride (none of them negative) and both bases on 16 bytes, extents
+// and indices in 32 bits.
 bool maxpool_cl_ok(const qa_maxpool_desc& d) {
     if (d.code != 1 && d.code != 2) return false;
     const int64_t ch = 16 / d.code, lim = (int64_t)1 << 30;
     const int64_t st[6] = {d.x_sn, d.x_sh, d.x_sw, d.y_sn, d.y_sh, d.y_sw};
     for (int64_t v : st)
-        if (v % ch) return false;
+        if (v < 0 || v % ch) return false;
     const int64_t ext[] = {d.H, d.W, d.KH, d.KW, d.C, d.KH * d.KW,
                            d.OH * d.SH, d.OW * d.SW, d.KH * d.DH,
                            d.KW * d.DW};
@@ -372,24 +390,31 @@ bool maxpool_cl_ok(const qa_maxpool_desc& d) {
            d.N * d.OH * d.OW * ceil_div(d.C, ch) < ((int64_t)1 << 31);
 }
 
+// Launches a 16-byte form, or leaves the pool to the element kernel: false.
 template <class T>
-void launch_maxpool_cl(const qa_maxpool_desc& d, hipStream_t st) {
-    const int64_t nch = ceil_div(d.C, 16 / (int64_t)sizeof(T));
+bool launch_maxpool_cl(const qa_maxpool_desc& d, hipStream_t st) {
+    constexpr int64_t ch = 16 / sizeof(T);
+    const int64_t nch = ceil_div(d.C, ch);
     const int64_t outs = d.N * d.OH * d.OW;
     // Many taps and few outputs: a work-group an output (taps without an
     // unrolled form in a thread, one after the other, against it, us: 64x512
     // of 7x7 -> 1x1 12.1 / 3.9, 4x4 windows of 32x256x32x32, 32768 chunks
-    // of outputs, 5.6 / 5.0, 7x7 of 16x128x20x20, 51200, 11.4 / 13.4).
+    // of outputs, 5.6 / 5.0, 7x7 of 16x128x20x20, 51200, 11.4 / 13.4; with a
+    // partial last chunk 4x4 of 4x15x21x21 4.1 / 4.9).
     const int64_t taps = d.KH * d.KW;
     const bool unrolled = d.KH == 5 && d.KW == 5;
     if ((taps >= 64 && outs * nch < 65536) ||
-        (taps >= 16 && !unrolled && outs * nch <= 32768)) {
+        (taps >= (d.C % ch ? 32 : 16) && !unrolled && outs * nch <= 32768)) {
         int cb = 1;
         while (cb < nch && cb < 16) cb *= 2;
         const dim3 g((unsigned)outs, (unsigned)ceil_div(nch, cb));
         k_maxpool_wide<T><<<g, kThreads, 0, st>>>(d, (uint32_t)nch, cb);
-        return;
+        return true;
     }
+    // A partial last chunk stores by elements: not for small maps (element
+    // kernel / this one, us: 4x15x41x41 5x5 5.5 / 8.2, 2x24x28x28 2x2 2.9 /
+    // 3.4; 8x100x20x20 5x5 7.2 / 6.1, 32x24x56x56 2x2 5.5 / 3.9).
+    if (d.C % ch && outs * d.C < (1 << 18)) return false;
     const int64_t total = outs * nch;
     const unsigned nb =
         (unsigned)std::min<int64_t>(ceil_div(total, kThreads), 1 << 20);
@@ -403,6 +428,7 @@ void launch_maxpool_cl(const qa_maxpool_desc& d, hipStream_t st) {
         k_maxpool_cl<T, 5><<<nb, kThreads, 0, st>>>(d, n32, t32);
     else
         k_maxpool_cl<T, 0><<<nb, kThreads, 0, st>>>(d, n32, t32);
+    return true;
 }
 
 bool code_ok(int64_t c) { return c == 1 || c == 2 || c == 4; }
@@ -499,13 +525,9 @@ QA_API int qa_d_maxpool(const qa_maxpool_desc* d, void* stream) {
         return -1;
     }
     hipStream_t st = (hipStream_t)stream;
-    if (maxpool_cl_ok(*d)) {
-        if (d->code == 1)
-            launch_maxpool_cl<int8_t>(*d, st);
-        else
-            launch_maxpool_cl<int16_t>(*d, st);
+    if (maxpool_cl_ok(*d) && (d->code == 1 ? launch_maxpool_cl<int8_t>(*d, st)
+                                           : launch_maxpool_cl<int16_t>(*d, st)))
         return launched("qa_d_maxpool") ? 0 : -1;
-    }
     const unsigned nb = blocks_for(total);
     switch (d->code) {
         case 1: k_maxpool<int8_t><<<nb, kThreads, 0, st>>>(*d, total); break;

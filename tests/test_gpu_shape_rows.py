@@ -35,7 +35,12 @@ def _dev(a):
     (2, 24, 11, 12, (4, 4), (2, 2), (1, 1), (1, 1)),
     (3, 33, 8, 9, (2, 8), (1, 1), (2, 1), (0, 2)),
     (9, 256, 17, 16, (4, 5), (1, 1), (1, 1), (2, 2)),  # 41472, 82944 chunks
-    (2, 16, 9, 9, (5, 3), (2, 2), (1, 1), (1, 1))])
+    (2, 16, 9, 9, (5, 3), (2, 2), (1, 1), (1, 1)),
+    # partial last chunks past the size from which they take chunks
+    (5, 100, 25, 24, (5, 5), (1, 1), (1, 1), (2, 2)),
+    (3, 33, 56, 57, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 24, 150, 150, (2, 2), (2, 2), (1, 1), (0, 0)),
+    (1, 36, 90, 91, (3, 2), (1, 1), (1, 1), (0, 1))])
 @pytest.mark.parametrize("high", [False, True])
 def test_maxpool_chunks(hip, code, n, c, h, w, k, s, dl, pad, high):
     t = TYPES[code]
