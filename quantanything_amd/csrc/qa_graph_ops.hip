@@ -645,12 +645,17 @@ QA_API int qa_d_gap(const void* x, int in_code, int64_t x_sn, int64_t x_sc,
     // 2x2 3.7 / 2.8, of 4x4 3.7 / 4.5, but 256x256 of 4x4 5.8 / 4.6), nor
     // where words of 4 channels fill the 256 CUs, most lanes busy (256x256 of
     // 28x28 23.4 / 19.8, 64x1280 27.2 / 22.5; 2048x64 31.2 / 38.6).
+    // A partial last chunk, read by elements, moves the lines (64x300 of
+    // 14x14 8.4 / 5.9, of 600 pixels 12.3 / 11.1, 1x20 of 28x28 7.2 / 13.8;
+    // 64x301 of 7x7 5.7 / 10.1 against a thread a channel).
+    const bool whole = C % ch == 0;
     if (words) {
         const int64_t wg = qa::ceil_div(C, 256);
-        rows16 = rows16 && HW > 128 &&
-                 !(C >= 192 * wg && N * wg >= 256);
+        rows16 = rows16 && HW > (whole ? 128 : 511) &&
+                 !(whole ? C >= 192 * wg && N * wg >= 256
+                         : C >= 128 * wg && N * wg >= 128);
     } else {
-        rows16 = rows16 && HW > 8 &&
+        rows16 = rows16 && HW > (whole ? 8 : 24) &&
                  !(HW <= 16 && N * qa::ceil_div(C, 4 * ch) >= 2048);
     }
     if (rows16) {

@@ -49,7 +49,9 @@ def test_gap_rows(hip, code, n, c, hw, fill):
 @pytest.mark.parametrize("n,c,hw,sp,off", [
     (3, 20, 49, 20, 0), (2, 64, 700, 68, 4), (1, 300, 3, 320, 12),
     (2, 12, 3136, 24, 12), (2, 4, 1, 4, 0), (300, 256, 130, 256, 0),
-    (3, 128, 128, 128, 0), (3, 128, 129, 128, 0),  # words of 4 channels
+    (3, 128, 128, 128, 0), (3, 128, 129, 128, 0), (3, 20, 511, 32, 0),
+    (3, 20, 512, 32, 0), (70, 300, 513, 304, 0),  # words of 4 channels
+    (3, 18, 24, 32, 0), (3, 18, 25, 32, 0),
     (2, 18, 49, 20, 0), (2, 20, 49, 21, 1), (2, 18, 8, 32, 0),
     (700, 130, 16, 144, 0)])  # a channel a thread
 def test_gap_words_and_channels(hip, n, c, hw, sp, off):
