@@ -149,7 +149,10 @@ def test_copy_rows(hip, code, shape, xst, yst, off):
     (77, 40, 64, 48, 1500000000, -1, -100, 90),
     (5, 16, 16, 16, 1 << 30, -1, -128, 127),
     (3, 1000, 1008, 1024, 2000000001, 3, -128, 127),
-    (4096, 17, 32, 32, -1100000000, 1, -128, 127)])
+    (4096, 17, 32, 32, -1100000000, 1, -128, 127),
+    # a partial last chunk past the size from which chunks pay
+    (16384, 17, 32, 48, -1100000000, 1, -128, 127),
+    (9000, 30, 32, 32, 1500000000, -1, -100, 90)])
 def test_rescale_rows(hip, rows, cols, xs, ys, m, s, qmin, qmax):
     rng = np.random.default_rng(cols)
     x = rng.integers(-128, 128, (rows, xs)).astype(np.int8)
