@@ -47,10 +47,13 @@ int fast_io_args(const ConvArgs& a, ConvArgs& b, int epi) {
     return epi;
 }
 
-// The 128 x 128 blocks of a GEMM; 0 below 96 columns, which would leave them
-// half empty.
+// The 128 x 128 blocks of a GEMM; 0 below 96 columns or 64 rows, which would
+// leave them half empty (8x4096x4096 13.7 us on 64 x 128 blocks, 8.0 on the
+// convolution's tiles, K split; 64x4096x4096 13.0 / 14.5).
 static int64_t big_blocks(const ConvArgs& b) {
-    return b.Cout < 96 ? 0 : ceil_div(b.M, 128) * ceil_div(b.Cout, 128);
+    return b.Cout < 96 || b.M < 64
+               ? 0
+               : ceil_div(b.M, 128) * ceil_div(b.Cout, 128);
 }
 
 // Tile choice (from measured sweeps over the channel-block width WM and
@@ -113,7 +116,9 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
     // Without a hint (times of a launch in a graph of them, us; blocks =
     // 16-row x 64-channel blocks):
     // * a GEMM or pointwise convolution the narrow kernel takes, up to 1024
-    //   blocks (2048 for K of 256 to 576): 4096x576x64 3.8 against 7.1 on the
+    //   blocks (2048 for K of 256 to 576
+    //   with the weights in fragment order, without it 1576x576x1152 8.8 us
+    //   against 5.8 staged): 4096x576x64 3.8 against 7.1 on the
     //   tiles below, 197x384x1152 3.6 / 6.4, 1024x1024x1024 6.6 / 6.5 on the
     //   staged blocks, which win past it (4096x576x1024 9.9 / 8.2); two
     //   row tiles a wave past 512 blocks (4096x576x256 5.1 / 5.6); below
@@ -134,7 +139,7 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
         const int K = a.KGp * 16;
         if (blocks <= 1024 ||
             (blocks <= 2048 &&
-             (a.Cout < 128 || (K >= 256 && K <= 576))))
+             (a.Cout < 128 || (a.wfrag && K >= 256 && K <= 576))))
             return launch_gemm_narrow(b, st, blocks > 512 ? 2 : 1);
     }
     if (pointwise && b.M > b.N && b.rowio &&

@@ -431,8 +431,9 @@ bool flags(const ConvArgs& b, hipStream_t st) {
 //   registers do not fit beside the 128 accumulators.
 // * 256 x 128 blocks that fill as much, from 1024 K-bytes: 8192x4096x1024
 //   36.9 / 43.6. At 384 K-bytes they gain nothing (6304x384x1152 9.0 / 8.9).
-// * 64 x 128 blocks up to half a CU a 128 x 128 block: 256x4096x4096 16.7 /
-//   24.4, 5000x3072x300 12.2 / 21.4, 2000x512x700 6.0 / 8.4.
+// * 64 x 128 blocks up to half a CU a 128 x 128 block (a partial column
+//   block counted by its columns: 12000x32x140 5.1 / 6.6): 256x4096x4096
+//   16.7 / 24.4, 5000x3072x300 12.2 / 21.4, 2000x512x700 6.0 / 8.4.
 // * else 128 x 128 (6304x384x1536 11.5 / 13.7 with 64 x 128; past half a
 //   block a CU the deeper pipeline gains with every operand in L2 alone:
 //   6304x1536x384 10.4 / 12.2, but 19.1 / 18.5 within a network).
@@ -450,7 +451,7 @@ bool launch_gemm_stage(const ConvArgs& b, hipStream_t st, int form) {
         else if (b.KGp >= 64 && fills(blocks(256, 128)))
             form = 18;
         else
-            form = 2 * blocks(128, 128) <= cus ? 16 : 3;
+            form = 2 * ceil_div(b.M, 128) * b.Cout <= 128 * cus ? 16 : 3;
     }
     switch (form) {
         case 16: return flags<64, 128, 2, 2, 6>(b, st);

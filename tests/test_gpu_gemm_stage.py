@@ -33,3 +33,27 @@ def test_staged_blocks_bit_exact(hip, m, k, n):
         np.testing.assert_array_equal(got[:m * n].reshape(m, n), want,
                                       err_msg=hex(code))
         assert (got[m * n:] == 77).all(), hex(code)
+
+
+@pytest.mark.parametrize("frag", [True, False])
+@pytest.mark.parametrize("m,k,n", [
+    (1, 1536, 2048), (63, 640, 2100), (64, 640, 2100), (40, 4096, 1000),
+    (1030, 576, 1156), (10049, 32, 140), (12000, 64, 260)])
+def test_default_choice_bit_exact(hip, m, k, n, frag):
+    """Sizes on each side of the lines between the tiles, the narrow kernel
+    and the blocks, without a tile code, with and without the weights in
+    fragment order."""
+    from quantanything_amd.workloads import GemmWorkload
+
+    w = GemmWorkload(seed=m + n, M=m, K=k, N=n)
+    if not frag:
+        w.d.w_frag = None
+    g = w.spec
+    acc = ((g["a"].astype(np.float64) - g["zp_in"]) @
+           g["w"].astype(np.float64)).astype(np.int64)  # exact below 2^53
+    t = 31 + g["shift"]
+    q = ((acc + g["bias"]) * g["mult"] + (1 << (t - 1))) >> t
+    want = (np.clip(q + g["zp_out"], g["qmin"], g["qmax"]) - 128)
+    w.launch()
+    got = w.y.cpu().numpy()
+    np.testing.assert_array_equal(got.reshape(m, n), want)
