@@ -307,13 +307,12 @@ __device__ __forceinline__ int64_t plan_fold(int64_t c, uint32_t corr, int m) {
 // A 4-channel word of a row that may start anywhere (the GPU reads and
 // writes unaligned words; rows of a matrix whose width is not a multiple of
 // 4 start off 4 bytes).
+typedef uint32_t word_any __attribute__((aligned(1)));
 __device__ __forceinline__ uint32_t word_load(const int8_t* p) {
-    uint32_t w;
-    __builtin_memcpy(&w, p, 4);
-    return w;
+    return *(const word_any*)p;
 }
 __device__ __forceinline__ void word_store(int8_t* p, uint32_t w) {
-    __builtin_memcpy(p, &w, 4);
+    *(word_any*)p = w;
 }
 
 // Low bytes of four table entries packed into one word (byte = 0), or their
