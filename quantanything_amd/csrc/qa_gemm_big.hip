@@ -223,10 +223,10 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
                     const int8_t* pr =
                         (const int8_t*)a.res + pq * a.res_pst + c0;
                     if (!CHK) {
-                        w = word_load(pr);
+                        w = word_load_args(pr);
                     } else if (pok) {
                         if (cfull) {
-                            w = word_load(pr);
+                            w = word_load_args(pr);
                         } else {
 #pragma unroll
                             for (int r = 0; r < 4; ++r)
@@ -261,8 +261,8 @@ __global__ __launch_bounds__(256) void k_gemm_big(ConvArgs a) {
                 int8_t* p2 = Y2 ? (int8_t*)a.y2 + pq * a.y2_pst + c0
                                 : nullptr;
                 if (!CHK || (pok && cfull)) {
-                    word_store(py, wy);
-                    if (Y2) word_store(p2, w2);
+                    word_store_args(py, wy);
+                    if (Y2) word_store_args(p2, w2);
                 } else if (pok) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)

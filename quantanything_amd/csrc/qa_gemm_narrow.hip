@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_gemm_narrow(
             auto put = [&](int8_t* d, uint32_t w)
                            __attribute__((always_inline)) {
                 if (cs + 3 < a.Cout) {
-                    word_store(d, w);
+                    word_store_args(d, w);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 3; ++r)

@@ -276,7 +276,7 @@ __global__ __launch_bounds__(
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
                     for (int u = 0; u < NT / 4; ++u)
-                        rn[ib][r][u] = word_load(
+                        rn[ib][r][u] = word_load_args(
                             (const int8_t*)a.res +
                             (p0 + 16 * (i0 + ib) + r) * a.res_pst + c0 +
                             64 * u);
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(
                             const int8_t* pr =
                                 (const int8_t*)a.res + p * a.res_pst + c;
                             if (cfull) {
-                                rv = word_load(pr);
+                                rv = word_load_args(pr);
                             } else {
 #pragma unroll
                                 for (int j = 0; j < 4; ++j)
@@ -358,8 +358,8 @@ __global__ __launch_bounds__(
                         int8_t* p2 =
                             Y2 ? (int8_t*)a.y2 + p * a.y2_pst + c : nullptr;
                         if (!CHK || (pok && cfull)) {
-                            word_store(py, wy);
-                            if (Y2) word_store(p2, w2);
+                            word_store_args(py, wy);
+                            if (Y2) word_store_args(p2, w2);
                         } else if (pok) {
 #pragma unroll
                             for (int j = 0; j < 4; ++j)
