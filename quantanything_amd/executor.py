@@ -524,12 +524,14 @@ class DeviceExecutor:
         return DeviceTensor.nd(buf, 0, shape, strides, self.code, self.so, qp)
 
     def _new_rows(self, name, shape, qp):
-        """A 2-D tensor ``name`` read by Gemms alone: int8 rows padded with
-        zeros to the 64-byte K-steps of the GEMM kernels (a dense tensor
-        otherwise, or where other readers may want it dense)."""
+        """A 2-D tensor ``name`` read by Gemms alone: int8 rows off the
+        16-byte grid of the GEMM kernels' loads padded with zeros to their
+        64-byte K-steps (a dense tensor otherwise, which a graph input is
+        quantized into at full rate, or where other readers may want it
+        dense)."""
         users = self._cons.get(name, [])
         if self.code != 1 or name in self.graph.outputs or not users or \
-                any(u.kind != "gemm" for u in users) or shape[1] % 64 == 0:
+                any(u.kind != "gemm" for u in users) or shape[1] % 16 == 0:
             return self._new(shape, qp)
         return self._padded_rows(shape, qp)
 

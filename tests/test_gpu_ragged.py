@@ -45,7 +45,8 @@ def _check(g, qt, shape, tmp_path, rows=None):
 @pytest.mark.parametrize("qt", ["int8", "uint8"])
 @pytest.mark.parametrize("m,sizes", [
     (1, [17, 5]), (65, [100, 77]), (33, [63, 65, 31]), (1100, [129, 140, 9]),
-    (7, [48, 64, 33]), (130, [1, 200])])
+    (7, [48, 64, 33]), (130, [1, 200]),
+    (9, [80, 48, 208, 17]), (300, [1040, 16])])  # rows of whole chunks, dense
 def test_odd_gemms(hip, tmp_path, qt, m, sizes):
     b = G.GraphBuilder(51)
     y = "x"
