@@ -719,9 +719,11 @@ class DeviceExecutor:
         for name in g.outputs:
             t = self.tensors[name]
             if len(t.shape) == 4 and t.nhwc and t.sc == 1 and \
-                    t.sp >= t.channels and name not in self.softmax_of and \
+                    t.sp >= t.channels and not t.row_major() and \
+                    name not in self.softmax_of and \
                     t.shape[0] * t.pixels < 2**31 - 4096:
                 # channels-last: dequantized into NCHW floats in one launch
+                # (where they are in row-major order, as any dense tensor)
                 yf = torch.empty(t.shape, dtype=torch.float32, device="cuda")
                 self.outputs_f32[name] = yf
                 self._add(f"dequantize:{name}", lambda s, t=t, yf=yf:
