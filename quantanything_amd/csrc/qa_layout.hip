@@ -296,7 +296,8 @@ bool dequantize_planes(const T* x, int64_t x_sn, int64_t x_sp, int64_t N,
     constexpr int CH = 16 / sizeof(T);
     const int64_t gx = ceil_div(N * HW, 256), gy = ceil_div(C, CH);
     if (!tile_grid_ok(N * HW, gy)) {
-        set_error("qa_d_dequantize_nchw", "2^31 pixels or more");
+        set_error("qa_d_dequantize_nchw",
+                  "2^31 pixels or more, or more than 65535 chunks of channels");
         return false;
     }
     const bool vec = x_sp % CH == 0 && x_sn % CH == 0 && (uintptr_t)x % 16 == 0;

@@ -721,7 +721,8 @@ class DeviceExecutor:
             if len(t.shape) == 4 and t.nhwc and t.sc == 1 and \
                     t.sp >= t.channels and not t.row_major() and \
                     name not in self.softmax_of and \
-                    t.shape[0] * t.pixels < 2**31 - 4096:
+                    t.shape[0] * t.pixels < 2**31 - 4096 and \
+                    t.channels <= 65535 * 8:
                 # channels-last: dequantized into NCHW floats in one launch
                 # (where they are in row-major order, as any dense tensor)
                 yf = torch.empty(t.shape, dtype=torch.float32, device="cuda")

@@ -92,3 +92,27 @@ def test_values_past_float32_quotients(hip, code, c, hw, sp, scale):
     want = (q.astype(np.int64) - so).astype(dt)
     got = y.cpu().numpy().reshape(2, hw, sp)
     np.testing.assert_array_equal(got[:, :, :c], want.transpose(0, 2, 1))
+
+
+@pytest.mark.parametrize("qt", ["int8", "int16"])
+def test_output_of_many_channels(hip, qt):
+    """More channels than the one-launch dequantization's grid takes: a
+    dense copy first."""
+    from quantanything_amd import graph as G
+    from quantanything_amd.container import QuantContainer
+    from quantanything_amd.synth import Stream
+
+    shape = (1, 65535 * 16 + 16, 2, 1)
+    b = G.GraphBuilder(3)
+    g = b.build("x", [None, *shape[1:]],
+                b.op("MaxPool", ["x"], kernel_shape=[1, 1], strides=[1, 1]))
+    data = Stream(4).normal(shape).astype(np.float32)
+    q = QuantContainer(g, qt, per_channel=True)
+    q.calibrate([data])
+    ex = q.executor({"x": shape})
+    out = ex.run({"x": data})[g.outputs[0]]
+    t = ex.tensors[g.outputs[0]]
+    v = np.clip(np.rint(data.astype(np.float64) / t.qp.scale) + t.qp.zp,
+                t.qp.qmin, t.qp.qmax)
+    np.testing.assert_array_equal(
+        out, ((v - t.qp.zp) * t.qp.scale).astype(np.float32))
