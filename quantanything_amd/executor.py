@@ -769,6 +769,16 @@ class DeviceExecutor:
             (groups == 1 or cg % 16 == 0 or layout == 2)
 
     @staticmethod
+    def _mfma_limits(geo):
+        """Whether a layer (the 16 geometry fields of its descriptor) is
+        within the int8 MFMA launches' 32-bit limits: below 2^31 output
+        pixels, taps displaced by less than 2^15."""
+        n, kh, kw, dh, dw, oh, ow = (geo[k] for k in (0, 5, 6, 11, 12, 14,
+                                                      15))
+        return n * oh * ow < 2**31 and (kh - 1) * dh < 32768 and \
+            (kw - 1) * dw < 32768
+
+    @staticmethod
     def _f64_ok(x, a_off):
         """16-bit activations the FP64 matrix-core path takes: channels
         contiguous, centred values within 2^17."""
@@ -874,7 +884,7 @@ class DeviceExecutor:
                     kh * kw <= 52 and x.sp >= -(-cout // 16) * 16 and \
                     (h + pads[0] + kh * dil[0]) * \
                     (w + pads[1] + kw * dil[1]) * x.sp < 2**30 and \
-                    max((kh - 1) * dil[0], (kw - 1) * dil[1]) < 32768:
+                    self._mfma_limits(geo):
                 layout = 2  # depthwise (the kernel's 32-bit offsets)
         else:
             k, ncol = layer.w_centered.shape
@@ -902,7 +912,8 @@ class DeviceExecutor:
             x = xc
         use_mfma = self._mfma_ok(layer, x, layout, groups, cg, cg * kh * kw)
         if not use_mfma and x.code == 1 and x.sc == 1 and layout != 1 and \
-                (len(x.shape) == 2 or x.channels > 4):
+                (len(x.shape) == 2 or x.channels > 4) and \
+                self._mfma_limits(geo):
             # rows or pixels off the 16-byte grid (odd features, channel
             # halves): one copy onto it, where nothing else is in the way
             probe = DeviceTensor(None, 0, (1, 16, 1, 1), 16, 1, 16, x.code,
