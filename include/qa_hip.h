@@ -295,7 +295,8 @@ int qa_plan_epilogue_i8(const qa_epi_params* p, void* plan);
  * 65,536 levels): writes a plan of qa_lut_i16_plan_bytes(lut_len) bytes,
  * whose device copy (16-byte aligned) a w_code 8 descriptor with that table
  * may carry as epi_plan; its launches then read the table from LDS where
- * that pays. Returns 1 when planned, 0 when the table is not smooth enough
+ * that pays (any other plan, and one of a table of another length, is
+ * ignored). Returns 1 when planned, 0 when the table is not smooth enough
  * (entries more than 2 below or 1 above the rounded line between every
  * 16th in more than two of its groups of 16) or spans more than 65,535, -1 on bad arguments (lut_len 1 to
  * 65,536). Results do not depend on it. */

@@ -51,14 +51,18 @@ struct BsEpi {
 
 constexpr int BIAS_LIM_LOG2 = 51;
 
-// A 16-bit activation table for LDS (qa_plan_lut_i16): {base, entries, two
-// groups}, then per group of 16 consecutive entries 8 bytes: the first entry
-// and the next group's first as uint16 above base, and 2 bits an entry, its
-// difference (+ 2) from the rounded line between them. A smooth table (SiLU
-// over 2^16 levels is within one step of those lines) then takes 32 KB
-// instead of 256 KB; up to two groups that are not (where the clip cuts in)
-// are named in the header, and their entries read from the table itself.
+// A 16-bit activation table for LDS (qa_plan_lut_i16): {base, entries with
+// the format's tag, two groups}, then per group of 16 consecutive entries 8
+// bytes: the first entry and the next group's first as uint16 above base, and
+// 2 bits an entry, its difference (+ 2) from the rounded line between them.
+// A smooth table (SiLU over 2^16 levels is within one step of those lines)
+// then takes 32 KB instead of 256 KB; up to two groups that are not (where
+// the clip cuts in) are named in the header, and their entries read from the
+// table itself.
 constexpr int LUTP_HEAD = 16;
+// In the entries' word, above their 17 bits: the kernel reads a plan only
+// when it is one, of a table as long as the descriptor's.
+constexpr int LUTP_TAG = 0x51a80000;
 
 __device__ __forceinline__ int lutp_get(const uint2* t, int base, int i) {
     const uint2 w = t[i >> 4];
@@ -136,12 +140,13 @@ __global__ __launch_bounds__(64 * BS_WAVES) void k_conv_bsl(ConvArgs a,
         }
     }
     int4 lhead = int4{0, 0, -1, -1};
-    if (lutp) {
+    if (lutp) {  // (the launcher found that many bytes readable there)
         const int8_t* src = (const int8_t*)a.plan + LUTP_HEAD;
         lhead = *(const int4*)a.plan;
         const int nc = (int)((a.lut_len + 15) / 16 + 1) / 2;  // of 16 bytes
         for (int c = tid; c < nc; c += 64 * BS_WAVES)
             ((int4*)s_lut)[c] = ((const int4*)src)[c];
+        if (lhead.y != (LUTP_TAG | (int)a.lut_len)) lutp = 0;
     }
     // the element offset of a k-group's 16 channels from the tap's input
     // pixel (-1: no tap), its displacement dy << 16 | dx
@@ -436,6 +441,21 @@ bool exact_mul(int64_t m, int64_t shift) {  // mul_d's range with tmax 53
            m < ((int64_t)1 << 31);
 }
 
+// Whether the bytes at p, wherever a caller's plan came from, lie in one
+// device allocation (a lookup in the runtime's map; memory it does not know
+// is left alone). The kernel requests them together with the header that
+// says whether they are a plan: a wait for it first costs 0.45 us a launch.
+bool readable(const void* p, int64_t bytes) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) !=
+        hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return (uintptr_t)p + bytes <= (uintptr_t)base + size;
+}
+
 double host_mul(int64_t m, int64_t shift) {
     return ldexp((double)m, -(int)(31 + shift));
 }
@@ -527,8 +547,10 @@ bool launch_conv_bsl(const ConvArgs& b0, bool narrow, int wm,
     const int64_t nwg = std::min<int64_t>(
         ceil_div(ntiles, BS_WAVES) * gy * b.G, 2 * (int64_t)cus);
     const int64_t lutb = round_up(ceil_div(b.lut_len, 16) * 8, 16);
-    const bool lutp = b.lut && b.plan && lds + lutb <= BSL_LDS_MAX &&
-                      b.M * b.Cout >= 4096 * nwg;
+    const bool lutp = b.lut && b.plan && (uintptr_t)b.plan % 16 == 0 &&
+                      b.lut_len <= 65536 && lds + lutb <= BSL_LDS_MAX &&
+                      b.M * b.Cout >= 4096 * nwg &&
+                      readable(b.plan, LUTP_HEAD + lutb);
     if (lutp) lds += lutb;
     // (see launch_kernel of the int8 form)
     b.xcd_yfast = 2 * (int64_t)b.N * b.H * b.W * b.Cg * b.G >=
@@ -596,7 +618,7 @@ QA_API int qa_plan_lut_i16(const int32_t* lut, int64_t lut_len, void* plan) {
     memset(plan, 0, (size_t)bytes);
     int32_t* head = (int32_t*)plan;
     head[0] = (int32_t)base;
-    head[1] = (int32_t)lut_len;
+    head[1] = LUTP_TAG | (int32_t)lut_len;
     head[2] = head[3] = -1;
     uint32_t* out = (uint32_t*)((char*)plan + LUTP_HEAD);
     int odd = 0;

@@ -63,3 +63,35 @@ def test_bit_exact(hip, tmp_path, n, cin, cout, k, stride, size, form):
                     err_msg=f"{name} {code:#x}")
                 checked += 1
         assert checked >= 1
+
+
+@pytest.mark.parametrize("other", ["shorter", "int8", "off 16"])
+def test_other_plans_are_ignored(hip, other):
+    """A descriptor whose epi_plan is not the plan of its own table (of a
+    shorter table, an int8 epilogue's, off its alignment) reads the table
+    itself."""
+    import torch
+
+    b = G.GraphBuilder(62)
+    y = b.silu(b.conv("x", 16, 32, 1, 1, w_scale=0.25))
+    shape = (9, 16, 66, 66)
+    g = b.build("x", [None, *shape[1:]], y)
+    q = QuantContainer(g, "int16", per_channel=True)
+    q.calibrate([Stream(12).normal((1,) + shape[1:]).astype(np.float32)])
+    data = Stream(13).normal(shape, 1.4).astype(np.float32)
+    ex = q.executor({"x": shape})
+    want = ex.run({"x": data})[g.outputs[0]].copy()
+    d, = [d for d in ex.keep if isinstance(d, ConvDesc)]
+    lib, n = hip.library(), int(d.lut_len)
+    assert d.epi_plan and n > 40
+    lut = np.arange(40 if other == "shorter" else n, dtype=np.int32)
+    plan = np.zeros(lib.qa_lut_i16_plan_bytes(len(lut)), np.uint8)
+    assert lib.qa_plan_lut_i16(lut.ctypes.data, len(lut),
+                               plan.ctypes.data) == 1
+    if other == "int8":  # its header: clip bounds, shift, flags
+        plan = np.zeros(64, np.uint8)
+        plan[:16].view(np.int32)[:] = (-128, 127, 1 << 16, 0)
+    dev = torch.from_numpy(np.concatenate(
+        [np.zeros(8 if other == "off 16" else 0, np.uint8), plan])).cuda()
+    d.epi_plan = dev.data_ptr() + (8 if other == "off 16" else 0)
+    np.testing.assert_array_equal(ex.run({"x": data})[g.outputs[0]], want)
