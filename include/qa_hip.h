@@ -244,7 +244,10 @@ typedef struct qa_conv_desc {
                       (2,1,0), (1,4,0), (1,1,1), (2,1,1), (4,1,1); tm =
                       16-pixel tiles per wave; with wsplit, 0x11000 | wm |
                       tm << 4 ((wm, tm) in {1, 2, 4} x {1, 2}) runs the
-                      byte-split form. Results do not depend on it. */
+                      byte-split form: with its weights in LDS where
+                      qa_conv_split_lds says so, tm then not looked at (nor
+                      wm, for at most 4 input channels). Results do not
+                      depend on it. */
     const void* wsplit;        /* w_code 8 only, optional: the same weights
                                   from qa_pack_weights_i16s (both planes);
                                   the int16 input then runs on the int8
@@ -290,6 +293,12 @@ typedef struct qa_epi_params {
 } qa_epi_params;
 int64_t qa_epi_plan_bytes(int64_t cout);
 int qa_plan_epilogue_i8(const qa_epi_params* p, void* plan);
+
+/* Which kernel the byte-split tile codes of a w_code 8 descriptor run: 1 the
+ * one with its weights in LDS (a code's channel block wm alone counts), 2
+ * the same for at most 4 input channels (every code is the same kernel), 0
+ * another, or none (host side, no GPU). */
+int qa_conv_split_lds(const qa_conv_desc* d);
 
 /* Host-side planner of a 16-bit activation table in its LDS form (32 KB for
  * 65,536 levels): writes a plan of qa_lut_i16_plan_bytes(lut_len) bytes,

@@ -189,6 +189,10 @@ bool mfma_launch_lds(const ConvArgs& b, int wm, bool split, int epi,
                      hipStream_t st);
 bool mfma_launch_l2(const ConvArgs& b, int wm, bool split, int epi,
                     hipStream_t st);
+// Which form the byte-split tile codes of a 16-bit descriptor run: 0 not the
+// LDS-resident one, 1 that one (of the code, its channel block alone counts),
+// 2 its narrow form (nothing of the code does).
+int conv_split_lds(const ConvArgs& a);
 bool launch_conv_valu(const ConvArgs& a, hipStream_t st);
 // Depthwise convolutions (layout 2; qa_conv_dw.hip); arguments in launch
 // form, `epi` as chosen by launch_conv_mfma.

@@ -605,6 +605,59 @@ constexpr F64Tile kF64Tiles[] = {
 
 }  // namespace
 
+// The launch form: whether the outputs are dense channels-last (fastio) and
+// their pixel strides.
+static ConvArgs f64_args(const ConvArgs& a) {
+    ConvArgs b = a;
+    {
+        // dense channels-last y (residual, copy): element of pixel p and
+        // channel c at p * pixel stride + c (a GEMM row is one pixel)
+        const int64_t ohw = (int64_t)a.OH * a.OW;
+        auto pst = [&](int64_t sn, int64_t sp) { return ohw == 1 ? sn : sp; };
+        auto dense = [&](const void* p, int64_t sn, int64_t sc, int64_t sp) {
+            return p == nullptr || (sc == 1 && (ohw == 1 || sn == ohw * sp));
+        };
+        b.fastio = dense(a.y, a.y_sn, a.y_sc, a.y_sp) &&
+                   dense(a.res, a.res_sn, a.res_sc, a.res_sp) &&
+                   dense(a.y2, a.y2_sn, a.y2_sc, a.y2_sp);
+        b.y_pst = pst(a.y_sn, a.y_sp);
+        b.res_pst = pst(a.res_sn, a.res_sp);
+        b.y2_pst = pst(a.y2_sn, a.y2_sp);
+    }
+    return b;
+}
+
+// The byte-split form on the int8 matrix cores: when the split planes are
+// given and the input fits it (16-byte aligned 16-channel groups, K' = 16 KGp
+// < 2^16, the stored zero point an int16). 0: not; 1: it takes the layer; 2:
+// in its narrow form (at most 4 channels in 8-byte aligned 4-channel pixels),
+// which has one 16-channel block a wave.
+static int split_form(const ConvArgs& a) {
+    const uintptr_t xa = (uintptr_t)a.x;
+    const bool narrow = a.Cg <= 4 && a.G == 1 && a.x_sp % 4 == 0 &&
+                        a.x_sn % 4 == 0 && xa % 8 == 0;
+    if (!(a.ws && a.ws_k &&
+          ((a.Cg % 16 == 0 && a.x_sp % 8 == 0 && a.x_sn % 8 == 0 &&
+            xa % 16 == 0) ||
+           narrow) &&
+          a.KGp > 0 && a.KGp < 4096 && a.x_add >= -32767 &&
+          a.x_add <= 32768 &&
+          // the k-group table's int32 offsets, displacements below 2^15 and
+          // every pixel base of the padded extent in int32
+          (int64_t)(a.H + a.PH + a.KH * a.DH + a.SH) *
+                      (a.W + a.PW + a.KW * a.DW + a.SW) * a.x_sp +
+                  16 * (int64_t)a.CB < ((int64_t)1 << 31) &&
+          (int64_t)(a.KH - 1) * a.DH < 32768 &&
+          (int64_t)(a.KW - 1) * a.DW < 32768))
+        return 0;
+    return narrow && a.Cg % 16 != 0 ? 2 : 1;
+}
+
+int conv_split_lds(const ConvArgs& a) {
+    const int form = split_form(a);
+    return form && conv_bsl_applies(f64_args(a)) ? form : 0;
+}
+
 bool launch_conv_f64(const ConvArgs& a, hipStream_t st) {
     if (a.M <= 0 || a.Cog <= 0) return true;
     if (a.x_code != 2 || a.x_sc != 1 || a.narrow16 || a.Cg < 1 ||
@@ -627,47 +680,15 @@ bool launch_conv_f64(const ConvArgs& a, hipStream_t st) {
            (a.Cg % v || a.x_sn % v || a.x_sp % v || xa % (2 * v) ||
             ((a.Cg + 4 * v - 1) / (4 * v)) * 4 * v != cg4))
         v = v == 8 ? 4 : 1;
-    ConvArgs b = a;
-    {
-        // dense channels-last y (residual, copy): element of pixel p and
-        // channel c at p * pixel stride + c (a GEMM row is one pixel)
-        const int64_t ohw = (int64_t)a.OH * a.OW;
-        auto pst = [&](int64_t sn, int64_t sp) { return ohw == 1 ? sn : sp; };
-        auto dense = [&](const void* p, int64_t sn, int64_t sc, int64_t sp) {
-            return p == nullptr || (sc == 1 && (ohw == 1 || sn == ohw * sp));
-        };
-        b.fastio = dense(a.y, a.y_sn, a.y_sc, a.y_sp) &&
-                   dense(a.res, a.res_sn, a.res_sc, a.res_sp) &&
-                   dense(a.y2, a.y2_sn, a.y2_sc, a.y2_sp);
-        b.y_pst = pst(a.y_sn, a.y_sp);
-        b.res_pst = pst(a.res_sn, a.res_sp);
-        b.y2_pst = pst(a.y2_sn, a.y2_sp);
-    }
+    const ConvArgs b = f64_args(a);
     const int64_t ntiles = ceil_div(a.M, 16);
-    // the byte-split form on the int8 matrix cores: when the split planes
-    // are given and the input fits it (16-byte aligned 16-channel groups,
-    // K' = 16 KGp < 2^16, the stored zero point an int16); tile code 0x1000
-    // | wm | tm << 4, by default the widest channel block, one tile a wave
-    // narrow: at most 4 channels in 8-byte aligned 4-channel pixels
-    const bool narrow = a.Cg <= 4 && a.G == 1 && a.x_sp % 4 == 0 &&
-                        a.x_sn % 4 == 0 && xa % 8 == 0;
-    if (a.ws && a.ws_k &&
-        ((a.Cg % 16 == 0 && a.x_sp % 8 == 0 && a.x_sn % 8 == 0 &&
-          xa % 16 == 0) ||
-         narrow) &&
-        a.KGp > 0 && a.KGp < 4096 && a.x_add >= -32767 &&
-        a.x_add <= 32768 &&
-        // the k-group table's int32 offsets, displacements below 2^15 and
-        // every pixel base of the padded extent in int32
-        (int64_t)(a.H + a.PH + a.KH * a.DH + a.SH) *
-                (a.W + a.PW + a.KW * a.DW + a.SW) * a.x_sp +
-                16 * (int64_t)a.CB < ((int64_t)1 << 31) &&
-        (int64_t)(a.KH - 1) * a.DH < 32768 &&
-        (int64_t)(a.KW - 1) * a.DW < 32768) {
+    // the byte split: tile code 0x1000 | wm | tm << 4, by default the widest
+    // channel block, one tile a wave
+    const int form = split_form(a);
+    if (form) {
         int code = 0x1010 | (a.Cog >= 64 ? 4 : a.Cog >= 32 ? 2 : 1);
         if (a.tile_hint & TILE_VALID) code = a.tile_hint & 0xffff;
-        // the narrow form has one 16-channel block a wave
-        const bool nform = narrow && a.Cg % 16 != 0;
+        const bool nform = form == 2;
         // the weights in LDS, wherever they fit (a tile code of this form
         // gives the channel block; one tile a wave)
         if ((code & 0xff00) == 0x1000 && conv_bsl_applies(b)) {

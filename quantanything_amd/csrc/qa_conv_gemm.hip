@@ -805,6 +805,11 @@ QA_API int qa_d_conv(const qa_conv_desc* d, void* stream_) {
     return launch_conv_valu(a, st) ? 0 : -1;
 }
 
+QA_API int qa_conv_split_lds(const qa_conv_desc* d) {
+    ConvArgs a;
+    return desc_args(d, a, "qa_conv_split_lds") == 3 ? conv_split_lds(a) : 0;
+}
+
 // Launch forms of two chained convolution descriptors that the fused
 // kernel takes, or false.
 static bool pair_args(const qa_conv_desc* d1, const qa_conv_desc* d2,

@@ -2304,9 +2304,14 @@ class DeviceExecutor:
         if d.w_code == 8:  # FP64 path: wm | tm << 4 | split << 8
             wm_max = 1 if cog <= 16 else 2 if cog <= 32 else 4
             out = [0] + [0x10000 | c for c in F64_TILES if c & 15 <= wm_max]
-            if d.wsplit:  # byte split: 0x1000 | wm | tm << 4
-                out += [0x11000 | wm | tm << 4 for tm in (1, 2)
-                        for wm in (1, 2, 4) if wm <= wm_max]
+            if d.wsplit:  # byte split: 0x1000 | wm | tm << 4, each kernel
+                # once (with the weights in LDS one tile a wave, and one
+                # channel block for the narrow inputs)
+                lds = native.library().qa_conv_split_lds(ctypes.byref(d))
+                out += [0x11000 | wm | tm << 4
+                        for tm in ((1,) if lds else (1, 2))
+                        for wm in ((1,) if lds == 2 else (1, 2, 4))
+                        if wm <= wm_max]
             return out
         wm_max = 1 if cog <= 16 else 2 if cog <= 32 else 4 if cog <= 64 else 8
         out = [0]

@@ -66,6 +66,7 @@ def _declare(lib):
         "qa_pack_weights_f64": (i32, [p] + [i64] * 6 + [p]),
         "qa_pack_weights_i16s": (i32, [p] + [i64] * 5 + [p, p]),
         "qa_d_conv": (i32, [p, p]),
+        "qa_conv_split_lds": (i32, [p]),
         "qa_d_quantize_conv": (i32, [p, p, f64, i64, i64, i64, p]),
         "qa_d_conv_pool": (i32, [p, p, p]),
         "qa_conv_pw_pool_supported": (i32, [p, p]),

@@ -4,6 +4,8 @@ large enough that a work-group stages the table, channel counts around the
 Add and a Concat copy, inputs past the calibrated range (table clips), all
 against the oracle bit for bit."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -95,3 +97,52 @@ def test_other_plans_are_ignored(hip, other):
         [np.zeros(8 if other == "off 16" else 0, np.uint8), plan])).cuda()
     d.epi_plan = dev.data_ptr() + (8 if other == "off 16" else 0)
     np.testing.assert_array_equal(ex.run({"x": data})[g.outputs[0]], want)
+
+
+@pytest.mark.parametrize("n,cin,cout,k,size,form", [
+    (3, 16, 18, 3, 13, "plain"), (2, 32, 34, 1, 12, "add"),
+    (2, 48, 22, 3, 11, "concat"), (3, 3, 18, 3, 15, "add"),
+    (2, 4, 10, 3, 14, "concat"),  # pixels of 4 channels
+    (1, 576, 20, 3, 7, "plain"), (1, 560, 32, 3, 6, "add")])
+def test_form_without_lds(hip, tmp_path, n, cin, cout, k, size, form):
+    """The byte split without its weights in LDS, where that form does not
+    apply (pixels off 4 channels, weights past the LDS): every tile code,
+    plain, with a residual Add and with a Concat copy."""
+    b = G.GraphBuilder(63)
+    x = b.op("Relu", [b.conv("x", 5, cin, 1)]) if cin > 4 else "x"
+    if form == "add":
+        r = b.op("Relu", [b.conv(x, cin, cout, 1)])
+    y = b.silu(b.conv(x, cin, cout, k, w_scale=(cin * k * k) ** -.5))
+    if form == "add":
+        y = b.op("Add", [r, y])
+    elif form == "concat":
+        y = b.op("Concat", [b.op("MaxPool", [y], kernel_shape=[1, 1],
+                                 strides=[1, 1]), y], axis=1)
+    shape = (n, 5 if cin > 4 else cin, size, size)
+    g = b.build("x", [None, *shape[1:]], y)
+    q = QuantContainer(g, "int16", per_channel=True)
+    q.calibrate([Stream(14).normal(shape).astype(np.float32)])
+    q.save(tmp_path / "q.json")
+    data = Stream(15).normal(shape, 1.3).astype(np.float32)
+    oracle = OraclePipeline(g, str(tmp_path / "q.json"))
+    oracle.run(data, keep=True)
+    ex = q.executor({"x": shape})
+    ds = [d for d in ex.keep if isinstance(d, ConvDesc) and d.wsplit and
+          d.KH == k and not
+          hip.library().qa_conv_split_lds(ctypes.byref(d))]
+    assert ds and all((d.res if form == "add" else d.y2 if form == "concat"
+                       else True) for d in ds[-1:])
+    for code in [0] + [0x11000 | wm | tm << 4 for tm in (1, 2)
+                       for wm in (1, 2, 4)]:
+        for d in ds:
+            d.tile = code
+        ex.run({"x": data})
+        checked = 0
+        for name, t in ex.tensors.items():
+            if name in oracle.env:
+                got = t.to_host()
+                np.testing.assert_array_equal(
+                    got, oracle.env[name].reshape(got.shape),
+                    err_msg=f"{name} {code:#x}")
+                checked += 1
+        assert checked >= 1
