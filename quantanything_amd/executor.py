@@ -1142,6 +1142,41 @@ class DeviceExecutor:
                           if r <= d.OH]
             self.tunables.append((fused, d, rows, fn))
 
+    @staticmethod
+    def pool_fusion_pays(d):
+        """Whether the convolution ``d`` and the global average pool of its
+        output run faster as one launch than as two. A work-group of the
+        fused launch computes a whole image over up to 128 channels, so its
+        time hardly depends on the batch until the work-groups fill the
+        chip, while that of two launches grows with it. Measured (us, fused /
+        two; 777 sizes of batch 1 to 1024):
+
+        * images of up to 25 KB and 256 pixels: fused (batch 32, 128 -> 256
+          channels 7x7 5.7 / 7.6, 14x14 9.9 / 10.5);
+        * larger ones, pointwise and within the launch's LDS: fused past a
+          batch that grows with the image and K (64 -> 128 at 20x20 batch 32
+          11.7 / 10.4, 64 11.8 / 12.3, 256 12.2 / 23.3; 128 -> 256 at 20x20
+          batch 32 15.2 / 12.7, 80 15.6 / 18.2), in one round of work-groups
+          where a CU holds one (384 -> 1280 at 10x10 batch 16 11.7 / 12.1, 32
+          21.7 / 13.3);
+        * else two launches (64 -> 64 3x3 at 20x20 53 / 12, 128 -> 256 at
+          56x56 batch 32 232 / 33)."""
+        pixels, rows = d.OH * d.OW, d.w_kgp * 16 + 16  # LDS bytes a row
+        if pixels <= 256 and pixels * d.C <= 25600:
+            return True
+        if not (d.KH == d.KW == d.SH == d.SW == 1 and d.PH == d.PW == 0 and
+                d.OH == d.H and d.OW == d.W and d.C % 16 == 0):
+            return False
+        block = 64 if d.Cout <= 64 or 128 * rows > 65536 else 128
+        lds = (block + pixels) * rows
+        if lds > 96 * 1024:
+            return False
+        if (160 * 1024) // (lds + 1024) < 2 and \
+                d.N * -(-d.Cout // block) > 256:
+            return False
+        return d.N * -(-d.Cout // 128) * 128 >= \
+            6 * pixels + 64 * min(d.w_kgp * 16, 128)
+
     def _fuse_pools(self, cons):
         """An int8 MFMA convolution (one group, table plan, no residual or
         second output) whose output only feeds a global average pool runs
@@ -1158,12 +1193,7 @@ class DeviceExecutor:
             if len(hits) != 1:
                 continue
             d, ln = hits[0]
-            # A work-group of the fused launch computes a whole image, so
-            # it pays for images of up to 25 KB and 256 pixels (batch 32,
-            # 128 -> 256 channels: 14x14 10.1 us against 10.6 us as two
-            # launches, 20x20 15.5 against 10.9, 56x56 232 against 33;
-            # 384 -> 1280: 7x7 11.3 against 12.8, 10x10 22.3 against 12.8)
-            if d.OH * d.OW > 256 or d.OH * d.OW * d.C > 25600:
+            if not self.pool_fusion_pays(d):
                 continue
             if not (d.epi_plan and d.G == 1 and d.w_layout == 0 and
                     not d.res and not d.y2 and d.y_code == 1 and

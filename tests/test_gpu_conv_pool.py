@@ -105,3 +105,28 @@ def test_pointwise_pair_pool_bit_exact(hip, tmp_path, quant_type, c0, c1,
     c.save(path)
     ints, _ = OraclePipeline(g, path).run(x)
     np.testing.assert_array_equal(got, ints[g.outputs[0]])
+
+
+@pytest.mark.parametrize("quant_type", ["int8", "uint8"])
+@pytest.mark.parametrize("n,cin,cout,size,fused", [
+    (70, 16, 80, 20, True), (40, 24, 512, 17, True), (130, 32, 96, 28, True),
+    (5, 16, 80, 20, False)])
+def test_large_images_at_large_batches(hip, tmp_path, quant_type, n, cin,
+                                       cout, size, fused):
+    """Images past 256 pixels run fused from the batch where that pays, and
+    as two launches below it, both bit for bit."""
+    g = _head(cin, cout, 1, size, True)
+    shape = (n, cin, size, size)
+    q = QuantContainer(g, quant_type, per_channel=True)
+    q.calibrate([Stream(3).normal((2,) + shape[1:]).astype(np.float32)])
+    q.save(tmp_path / "q.json")
+    data = Stream(4).normal(shape, 1.1).astype(np.float32)
+    oracle = OraclePipeline(g, str(tmp_path / "q.json"))
+    oracle.run(data, keep=True)
+    ex = q.executor({"x": shape})
+    assert any(name.startswith("convpool:") for name, _ in ex.launches) == \
+        fused
+    ex.run({"x": data})
+    got = ex.integer_outputs()[g.outputs[0]]
+    np.testing.assert_array_equal(
+        got, oracle.env[g.outputs[0]].reshape(got.shape))
