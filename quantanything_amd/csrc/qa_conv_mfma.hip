@@ -49,11 +49,14 @@ int fast_io_args(const ConvArgs& a, ConvArgs& b, int epi) {
 
 // The 128 x 128 blocks of a GEMM; 0 below 96 columns or 64 rows, which would
 // leave them half empty (8x4096x4096 13.7 us on 64 x 128 blocks, 8.0 on the
-// convolution's tiles, K split; 64x4096x4096 13.0 / 14.5).
+// convolution's tiles, K split; 64x4096x4096 13.0 / 14.5), and for a short
+// product with a residual over few rows (1020x256x256 6.7 / 5.6, 1020x384x384
+// 7.2 / 6.7, 197x64x1024 5.3 / 4.9; 1020x768x768 8.1 / 11.5).
 static int64_t big_blocks(const ConvArgs& b) {
-    return b.Cout < 96 || b.M < 64
-               ? 0
-               : ceil_div(b.M, 128) * ceil_div(b.Cout, 128);
+    if (b.Cout < 96 || b.M < 64 ||
+        (b.res && b.M < 1024 && b.KGp <= 24))
+        return 0;
+    return ceil_div(b.M, 128) * ceil_div(b.Cout, 128);
 }
 
 // Tile choice (from measured sweeps over the channel-block width WM and
@@ -169,9 +172,10 @@ bool launch_conv_mfma(const ConvArgs& a, hipStream_t st) {
     while (wm > 1 && waves(wm, false) < want) wm >>= 1;
     bool split = a.layout == 0 && KS >= 4 && waves(wm, false) < simds / 2;
     // up to a wave a SIMD, K split over 32-channel blocks keeps the waves
-    // and halves a wave's steps (64x4096x4096 21.1 -> 14.8 us)
+    // and halves a wave's steps (64x4096x4096 21.1 -> 14.8 us; from 8 steps:
+    // 3000x512x64 6.4 -> 6.2, but 3000x256x64 5.3 -> 5.4)
     // (wave 0 alone finishes a split tile: not with the 128-bit epilogue)
-    if (epi == Q8_TABLE && a.layout == 0 && KS >= 4 && !split && wm == 1 &&
+    if (epi == Q8_TABLE && a.layout == 0 && KS >= 8 && !split && wm == 1 &&
         a.Cog > 16 && waves(1, false) <= simds) {
         wm = 2;
         split = true;

@@ -57,3 +57,30 @@ def test_default_choice_bit_exact(hip, m, k, n, frag):
     w.launch()
     got = w.y.cpu().numpy()
     np.testing.assert_array_equal(got.reshape(m, n), want)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1020, 256, 260), (1023, 384, 384), (1024, 384, 384), (197, 64, 1028),
+    (600, 448, 512), (3000, 448, 64), (3000, 512, 64)])
+def test_default_choice_with_a_residual(hip, m, k, n):
+    """The same lines for products with a residual, whose blocks pay later."""
+    import torch
+
+    from quantanything_amd.workloads import GemmWorkload
+
+    w = GemmWorkload(seed=m + n, M=m, K=k, N=n)
+    g, d = w.spec, w.d
+    r = np.random.default_rng(m).integers(-128, 128, (m, n)).astype(np.int8)
+    rd = torch.from_numpy(r).cuda()
+    d.res, d.res_sn, d.res_sc, d.res_so = rd.data_ptr(), n, 1, 128
+    d.za, d.ma, d.sa = 128, 1 << 30, -1  # both operands as they are
+    d.zb, d.mb, d.sb = 128, 1 << 30, -1
+    d.add_sign, d.add_zp, d.add_qmax = 1, 128, 255
+    w._plan(d, g["mult"], g["shift"], g["bias"])
+    acc = (g["a"].astype(np.int64) - g["zp_in"]) @ g["w"].astype(np.int64)
+    t = 31 + g["shift"]
+    q = ((acc + g["bias"]) * g["mult"] + (1 << (t - 1))) >> t
+    q = np.clip(q + g["zp_out"], g["qmin"], g["qmax"])
+    want = np.clip((q - 128) + r + 128, 0, 255) - 128
+    w.launch()
+    np.testing.assert_array_equal(w.y.cpu().numpy().reshape(m, n), want)
