@@ -38,9 +38,9 @@ def _dev(a):
     (2, 16, 9, 9, (5, 3), (2, 2), (1, 1), (1, 1)),
     # partial last chunks past the size from which they take chunks
     (5, 100, 25, 24, (5, 5), (1, 1), (1, 1), (2, 2)),
-    (3, 33, 56, 57, (3, 3), (1, 1), (1, 1), (1, 1)),
-    (2, 24, 150, 150, (2, 2), (2, 2), (1, 1), (0, 0)),
-    (1, 36, 90, 91, (3, 2), (1, 1), (1, 1), (0, 1))])
+    (4, 33, 56, 57, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (3, 24, 151, 150, (2, 2), (2, 2), (1, 1), (0, 0)),
+    (1, 36, 110, 111, (3, 2), (1, 1), (1, 1), (0, 1))])
 @pytest.mark.parametrize("high", [False, True])
 def test_maxpool_chunks(hip, code, n, c, h, w, k, s, dl, pad, high):
     t = TYPES[code]
