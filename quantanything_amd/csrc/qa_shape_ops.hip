@@ -402,7 +402,8 @@ bool launch_maxpool_cl(const qa_maxpool_desc& d, hipStream_t st) {
     // of outputs, 5.6 / 5.0, 7x7 of 16x128x20x20, 51200, 11.4 / 13.4; with a
     // partial last chunk 4x4 of 4x15x21x21 4.1 / 4.9).
     const int64_t taps = d.KH * d.KW;
-    const bool unrolled = d.KH == 5 && d.KW == 5;
+    const bool unrolled =
+        d.KH == d.KW && (d.KH == 2 || d.KH == 3 || d.KH == 5);
     if ((taps >= 64 && outs * nch < 65536) ||
         (taps >= (d.C % ch ? 32 : 16) && !unrolled && outs * nch <= 32768)) {
         int cb = 1;
@@ -416,6 +417,11 @@ bool launch_maxpool_cl(const qa_maxpool_desc& d, hipStream_t st) {
     // 3.4, 275 thousand outputs of 67 channels 2x2 3.2 / 3.4; 8x100x20x20 5x5
     // 7.2 / 6.1, 32x24x56x56 2x2 5.5 / 3.9).
     if (d.C % ch && outs * d.C < (taps >= 16 ? 1 << 18 : 3 << 17))
+        return false;
+    // Nor does a window without an unrolled form over a small map (3x64x37x37
+    // 2x3 3.2 / 3.5, 1x32x20x20 3x5 3.9 / 4.8; 8x64x37x37 2x3 3.7 / 3.6,
+    // int16 3x64x37x37 3.3 / 3.4).
+    if (!unrolled && outs * d.C < (sizeof(T) == 1 ? 5 << 15 : 1 << 15))
         return false;
     const int64_t total = outs * nch;
     const unsigned nb =
