@@ -1,8 +1,9 @@
 """GlobalAveragePool over 16-byte rows (qa_d_gap: whole and partial channel
 chunks, few and many pixels, extremes of int8 and int16) against NumPy and
 Python integers, and pointwise convolutions run as GEMMs over their pixels
-(large-GEMM blocks: partial row and column blocks, a residual, a Concat copy)
-against the oracle, every value equal."""
+(the narrow kernel below 1024 of its blocks, the large-GEMM blocks past that
+or with a residual: partial row and column blocks, a Concat copy) against the
+oracle, every value equal."""
 
 import numpy as np
 import pytest
@@ -81,7 +82,8 @@ def test_gap_words_and_channels(hip, n, c, hw, sp, off):
 @pytest.mark.parametrize("qt", ["int8", "uint8"])
 @pytest.mark.parametrize("cin,cout,size,form", [
     (64, 128, 19, "plain"), (128, 132, 16, "add"), (64, 200, 18, "concat"),
-    (192, 130, 17, "plain")])
+    (192, 130, 17, "plain"),
+    (64, 128, 46, "plain"), (64, 200, 47, "concat"), (192, 130, 38, "plain")])
 def test_pointwise_as_gemm(hip, tmp_path, qt, cin, cout, size, form):
     b = G.GraphBuilder(43)
     x = b.op("Relu", [b.conv("x", 4, cin, 1)])

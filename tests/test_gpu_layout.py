@@ -14,7 +14,7 @@ CODES = {1: (np.int8, 128, 0, 255), 2: (np.int16, 32768, 0, 65535)}
 
 @pytest.mark.parametrize("code,n,c,hw,sp,shift", [
     (1, 1, 5, 1, 16, 0), (1, 2, 24, 57 * 57, 32, 0), (1, 3, 16, 12, 16, 0),
-    (1, 8, 64, 56 * 56, 64, 0),  # four pixels a thread
+    (1, 8, 64, 56 * 56, 64, 0),
     (1, 2, 7, 9, 7, 0), (1, 2, 20, 10, 21, 1),  # element stores
     (2, 3, 3, 224 * 224, 4, 0), (2, 2, 9, 25, 9, 0),
     (2, 6, 3, 224 * 224, 4, 0), (2, 340, 1, 784, 4, 0),  # four pixels

@@ -184,15 +184,15 @@ def _gemm_block_graph(k, n, act, residual):
     (1500, 384, 1152, False, False),   # QKV-like, partial row block
     (1100, 256, 384, True, False),     # fc1-like with the Gelu table
     (1030, 1536, 200, False, True),    # fc2-like, residual, partial column block
-    (2048, 320, 256, True, True),      # 64-byte K steps (K / 64 odd)
+    (2048, 320, 256, True, True),      # five K steps
     (1024, 128, 256, False, False),    # two K steps: fewer than the stages
 ])
 def test_large_gemm_kernel_bit_exact(hip, tmp_path, quant_type, m, k, n, act,
                                      residual):
-    """Weight GEMMs of >= 1024 rows (the 128 x 128 block kernel, tile code
-    0x10400 with register-staged K steps, 0x10403 / 0x10404 with 3 / 4 LDS
-    stages filled by direct loads, and every other tile code) equal the
-    oracle bit for bit."""
+    """Weight GEMMs of >= 1024 rows (tile code 0x10400, the library's choice
+    of block, 0x10403 / 0x10404, 128 x 128 blocks with 3 / 4 LDS stages
+    filled by direct loads, and every other tile code) equal the oracle bit
+    for bit."""
     g = _gemm_block_graph(k, n, act, residual)
     calib = [Stream(90 + i).normal((256, k)).astype(np.float32)
              for i in range(2)]
