@@ -7,10 +7,14 @@
 // MFMAs run: with the reads of a step before its own MFMAs, a block alone on
 // its CU took about 850 cycles a step, most of them those reads.
 //
-// What bounds it: the LDS port. At 128 bytes a cycle a step of a 4-wave block
-// of 128 x 128 reads for 256 cycles and is filled in 128, its MFMAs take 256;
-// a 256 x 256 block of 8 waves takes 768 + 256 against 1024 (16384x1024x1024:
-// 28.3 us in 128 x 128 blocks, 21.5 here: 1600 TOP/s).
+// What bounds it: no one unit. 16384x1024x1024 takes 28.3 us in 128 x 128
+// blocks and 21.5-22.3 here (1540-1600 TOP/s), one block of 256 x 256 and 8
+// waves on each CU. Counted there: a wave lives 37.7 k cycles and waits 11.8 k
+// of them (direct loads, LDS, barriers); its SIMD's matrix core works 16.4 k;
+// the LDS is busy 6.2 k without a bank conflict, and a wave waits 1.0 k to
+// issue to it. Of the wave's 1762 VALU instructions 512 are MFMAs, most of the
+// rest its epilogue of 128 accumulators a lane, and no other block is on the
+// CU whose MFMAs could fill that time or the first stages' loads.
 //
 // The epilogue is the int8 table plan of qa_conv.h, identical in results to
 // the convolution kernel's; residual, copy and pixel sums are template flags,
